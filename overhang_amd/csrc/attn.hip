@@ -32,7 +32,8 @@
 #include "omh_internal.h"
 #include "omh_device.h"
 
-#include <math.h>
+#include <algorithm>
+#include <cmath>
 
 namespace omh {
 namespace {
@@ -802,274 +803,523 @@ void attn_flash_kernel(const AttnArgs a) {
     }
 }
 
-// The same flash attention with every product as three bf16 products on
-// the bf16 matrix cores (v_mfma_f32_16x16x32_bf16, fp32 accumulation): each
-// fp32 operand x splits as hi = bf16(x), lo = bf16(x - hi), so
+// The default flash attention, on the bf16 matrix cores
+// (v_mfma_f32_32x32x16_bf16, fp32 accumulation) with every product as three:
+// each fp32 operand x splits as hi = bf16(x), lo = bf16(x - hi), so
 // x = hi + lo to 2^-16 relative, and a.b = hi.hi + hi.lo + lo.hi with the
-// dropped lo.lo term below 2^-16 |a||b|; per 32 keys a wave issues 96 such
-// products against 256 fp32 ones.  K is staged into LDS as hi / lo planes
-// row-major (32 head dims per 16-byte read), V transposed (V^T[dim][key],
-// 8 keys per 16-byte read) with its keys in the order the probabilities
-// already sit in the score product's registers: position 8 g + j of a
-// V^T row holds key 16 (j / 4) + 4 g + j % 4, which lane group g of the
-// B operand P^T holds as register j % 4 of its score sub-tile j / 4.  Rows
-// are padded so that every 16-lane group's reads fall in distinct banks.
+// dropped lo.lo term below 2^-16 |a||b|.
+//
+// A wave owns one unit, 32 consecutive tokens of one query head, with q and
+// the output (128 registers each at HD = 256) in registers; a workgroup is 4
+// waves, one per SIMD, and 4 units of one kv group (the group's heads of a
+// token block, then the next block).  What bounds the kernel is the matrix
+// cores against the LDS reads of the K and V tiles: per 32-key tile a wave
+// reads the whole 64 KiB and issues 96 products of 32 cycles, 256 KiB per CU
+// (2048 cycles at 128 B per clock) against 3072 cycles of products on every
+// SIMD.  (16-token units on 8 waves, the form before, read 512 KiB per tile.)
+//
+// Tiles sit in LDS in MFMA operand order: fragment f is the 1 KiB that the
+// 64 lanes of one A operand read as 16 contiguous bytes each, so no read has
+// a bank conflict and no padding is needed.  K fragment (s, plane): lane l
+// holds key l % 32 at dims 16 s + 8 (l / 32) + j.  The score product S^T =
+// K Q^T leaves token l % 32, key 8 (i / 4) + 4 (l / 32) + i % 4 in register i,
+// which P^T as the B operand of O^T = V^T P^T takes as it stands (16-key step
+// u: registers 8 u + j), so V fragment (d / 2, u, d % 2, plane) holds, in lane l, dim
+// 32 d + l % 32 at the keys 16 u + 8 (j / 4) + 4 (l / 32) + j % 4.
+//
+// K runs one tile ahead of V: an iteration forms the next tile's scores, then
+// adds its own tile's P V while the next tile's softmax (VALU) runs beside
+// those products.  One barrier per tile.
+//
+// Steps whose units leave CUs idle (a turn appended to a long conversation)
+// split the keys over ns workgroups per unit group (attn_flash_plan); each
+// writes its unnormalised output, and attn_flash_merge_kernel merges them.
 template <int HD>
 struct Flash3Shape {
     static constexpr int KT = 32;                  // keys per tile
-    // bytes of one bf16 K row.  The padding sets the LDS bank conflicts of the
-    // 16-byte K reads (SQ_LDS_BANK_CONFLICT per T = 4096 dispatch at HD = 256):
-    // 270.5 M cycles unpadded, 67.6 M with 16 / 48 / 64 bytes, 33.8 M with 32
-    // or 96 bytes; 96 gave the fastest kernel (499-505 against 521-527 us
-    // under the counters, the fastest of seven calls 539 against 554 us);
-    // the two stages then take 156 KiB of LDS.
-    static constexpr int KLD = 2 * HD + 96;
-    static constexpr int VLD = 2 * KT + 16;        // bytes of one bf16 V^T row
-    static constexpr int KPL = KT * KLD, VPL = HD * VLD;
-    static constexpr int STAGE = 2 * KPL + 2 * VPL;   // K hi, K lo, V^T hi, V^T lo
-    static constexpr size_t LDS = 2 * (size_t)STAGE;
-    static constexpr int NS = HD / 32;             // 32-dim steps of q.k
-    static constexpr int NJ = HD / 16;             // 16-dim output tiles
-    static constexpr int PK = KT * HD / 4 / (8 * OMH_WAVE);         // K float4 pieces per thread
-    static constexpr int PV = KT / 2 * HD / 4 / (8 * OMH_WAVE);     // V (key pair, 4 dims) units per thread
-    static_assert(LDS <= 160 * 1024 && KLD % 16 == 0 && VLD % 16 == 0, "two stages in a CU's LDS, 16-byte rows");
+    static constexpr int NW = 4;                   // waves (units) per workgroup
+    static constexpr int NS = HD / 16;             // 16-dim steps of q.k
+    static constexpr int ND = HD / 32;             // 32-dim output tiles
+    static constexpr int KB = NS * 2 * 1024;       // bytes of a tile's K fragments: (s, plane)
+    static constexpr int VB = ND * 2 * 2 * 1024;   // of its V fragments: (d / 2, u, d % 2, plane)
+    static constexpr int TILE = KB + VB;           // a tile image: K, then V
+    static constexpr size_t LDS = 2 * (size_t)TILE;   // two K stages, then two V stages
+    static constexpr int EU = HD > 128 ? 1 : 2;    // waves per SIMD the registers allow
+    static_assert(LDS <= 160 * 1024 && KB == VB, "two stages in a CU's LDS");
 };
 typedef __bf16 omh_v8bf __attribute__((ext_vector_type(8)));
+typedef float omh_v16f __attribute__((ext_vector_type(16)));
 
-__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)a) | (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)b) << 16;
+// a and b as bf16 pairs: *hi = their roundings, *lo = the roundings of what those leave
+__device__ __forceinline__ void bf16_split2(float a, float b, uint32_t &hi, uint32_t &lo) {
+    typedef __bf16 v2bf __attribute__((ext_vector_type(2)));
+    hi = __builtin_bit_cast(uint32_t, v2bf{(__bf16)a, (__bf16)b});
+    const float ra = a - __builtin_bit_cast(float, hi << 16), rb = b - __builtin_bit_cast(float, hi & 0xffff0000u);
+    lo = __builtin_bit_cast(uint32_t, v2bf{(__bf16)ra, (__bf16)rb});
 }
-__device__ __forceinline__ float bf16_rest(float x) { return x - (float)(__bf16)x; }
+typedef uint32_t omh_v4u32 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void bf16_split8(const float (&v)[8], omh_v8bf &hi, omh_v8bf &lo) {
+    omh_v4u32 h, l;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        uint32_t x, y;
+        bf16_split2(v[2 * j], v[2 * j + 1], x, y);
+        h[j] = x;
+        l[j] = y;
+    }
+    hi = __builtin_bit_cast(omh_v8bf, h);
+    lo = __builtin_bit_cast(omh_v8bf, l);
+}
 
-// One 32-key tile of K and V on its way to the flash kernel's LDS image: the
-// fp32 rows of keys kt .. kt + 31 (past nkeys, the tile's first row again)
-// into registers (load), then as bf16 hi / lo planes, K by rows and V
-// transposed, in the Flash3Shape stage layout (put: to an LDS stage, or to
-// a tile image in memory that the kernel later copies into LDS whole).
+// K or V fragments of the tile of keys kt .. kt + 31 on their way to LDS (or
+// to a tile image in memory), 4 waves: wave w takes fragment pairs (hi, lo)
+// w, w + 4, ...  Rows past nkeys repeat the tile's first row, so every value
+// is a visible one.
 template <int HD>
-struct Flash3Tile {
+struct Flash3Frags {
     using F = Flash3Shape<HD>;
-    static constexpr int KT = F::KT, KLD = F::KLD, VLD = F::VLD, NT = 8 * OMH_WAVE;
-    omh_v4f kr[F::PK], vr[F::PV][2];
-    // V unit e: the key pair at V^T positions 2 pp, 2 pp + 1 (pp = e % 16) for
-    // head dims 4 c .. 4 c + 3 (c = e / 16), so the 16 lanes of a position
-    // pair sweep write one 64-byte run of a V^T row: no bank conflicts.
-    // Position 8 g + j holds key 16 (j / 4) + 4 g + j % 4.
-    static __device__ __forceinline__ int vkey(int pp) {
-        const int pos = 2 * pp, g8 = pos / 8, j = pos % 8;
-        return 16 * (j / 4) + 4 * g8 + j % 4;
-    }
-    __device__ __forceinline__ void load(const float *Kg, const float *Vg, int kt, int nkeys, int tid) {
-        auto key_of = [&](int kk) { return (size_t)(kt + kk < nkeys ? kt + kk : kt); };
+    static constexpr int N = F::NS / F::NW;        // fragment pairs per wave (of K, and of V)
+    static_assert(F::NS % F::NW == 0 && F::NS == 2 * F::ND, "whole fragments per wave");
+    float x[N][8];
+    __device__ __forceinline__ void load_k(const float *Kg, int kt, int nkeys, int w, int lane) {
+        const int kk = kt + lane % 32 < nkeys ? kt + lane % 32 : kt;
 #pragma unroll
-        for (int i = 0; i < F::PK; i++) {
-            const int e = tid + NT * i, kk = e / (HD / 4), c = e % (HD / 4);
-            kr[i] = *reinterpret_cast<const omh_v4f *>(Kg + key_of(kk) * HD + 4 * c);
-        }
+        for (int i = 0; i < N; i++) {
+            const float *src = Kg + (size_t)kk * HD + 16 * (w + F::NW * i) + 8 * (lane / 32);
+            const omh_v4f a = *reinterpret_cast<const omh_v4f *>(src), b = *reinterpret_cast<const omh_v4f *>(src + 4);
 #pragma unroll
-        for (int i = 0; i < F::PV; i++) {
-            const int e = tid + NT * i, k0 = vkey(e % 16), c = e / 16;
-            vr[i][0] = *reinterpret_cast<const omh_v4f *>(Vg + key_of(k0) * HD + 4 * c);
-            vr[i][1] = *reinterpret_cast<const omh_v4f *>(Vg + key_of(k0 + 1) * HD + 4 * c);
-        }
-    }
-    __device__ __forceinline__ void put(unsigned char *st, int tid) const {
-        unsigned char *Kh = st, *Kl = st + F::KPL, *Vh = st + 2 * F::KPL, *Vl = Vh + F::VPL;
-#pragma unroll
-        for (int i = 0; i < F::PK; i++) {
-            const int e = tid + NT * i, kk = e / (HD / 4), c = e % (HD / 4);
-            const omh_v4f x = kr[i];
-            uint2 hi, lo;
-            hi.x = bf16_pair(x[0], x[1]);
-            hi.y = bf16_pair(x[2], x[3]);
-            lo.x = bf16_pair(bf16_rest(x[0]), bf16_rest(x[1]));
-            lo.y = bf16_pair(bf16_rest(x[2]), bf16_rest(x[3]));
-            *reinterpret_cast<uint2 *>(Kh + kk * KLD + 8 * c) = hi;
-            *reinterpret_cast<uint2 *>(Kl + kk * KLD + 8 * c) = lo;
-        }
-#pragma unroll
-        for (int i = 0; i < F::PV; i++) {
-            const int e = tid + NT * i, pos = 2 * (e % 16), c = e / 16;
-#pragma unroll
-            for (int d = 0; d < 4; d++) {
-                const float x0 = vr[i][0][d], x1 = vr[i][1][d];
-                *reinterpret_cast<uint32_t *>(Vh + (4 * c + d) * VLD + 2 * pos) = bf16_pair(x0, x1);
-                *reinterpret_cast<uint32_t *>(Vl + (4 * c + d) * VLD + 2 * pos) = bf16_pair(bf16_rest(x0), bf16_rest(x1));
+            for (int j = 0; j < 4; j++) {
+                x[i][j] = a[j];
+                x[i][4 + j] = b[j];
             }
+        }
+    }
+    __device__ __forceinline__ void load_v(const float *Vg, int kt, int nkeys, int w, int lane) {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            const int f = w + F::NW * i, d = 2 * (f / 4) + f % 2, u = f / 2 % 2;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int k = kt + 16 * u + 8 * (j / 4) + 4 * (lane / 32) + j % 4;
+                x[i][j] = Vg[(size_t)(k < nkeys ? k : kt) * HD + 32 * d + lane % 32];
+            }
+        }
+    }
+    // (the pairs' order is the fragments': (s, plane) and (d / 2, u, d % 2, plane))
+    __device__ __forceinline__ void put(unsigned char *dst, int w, int lane) const {
+#pragma unroll
+        for (int i = 0; i < N; i++) {
+            omh_v8bf hi, lo;
+            bf16_split8(x[i], hi, lo);
+            unsigned char *p = dst + (size_t)(w + F::NW * i) * 2048 + 16 * lane;
+            *reinterpret_cast<omh_v8bf *>(p) = hi;
+            *reinterpret_cast<omh_v8bf *>(p + 1024) = lo;
         }
     }
 };
 
 // The tile images of keys 0 .. pos + T - 1 of the step's sequence, one
 // workgroup per (kv head, tile): image (g, i) at a.img + (g * a.img_tiles +
-// i) * STAGE holds exactly what attn_flash3_kernel stages in LDS for tile i.
+// i) * TILE holds exactly what attn_flash3_kernel stages in LDS for tile i.
 template <int HD>
-__global__ __launch_bounds__(8 * OMH_WAVE) void attn_tile_image_kernel(const AttnArgs a) {
+__global__ __launch_bounds__(Flash3Shape<HD>::NW * OMH_WAVE) void attn_tile_image_kernel(const AttnArgs a) {
     using F = Flash3Shape<HD>;
     const int g = blockIdx.x % a.KV, ti = blockIdx.x / a.KV;
-    const size_t cache0 = ((size_t)a.seq * a.KV + g) * a.max_t;
-    Flash3Tile<HD> t;
-    t.load(a.Kc + cache0 * HD, a.Vc + cache0 * HD, ti * F::KT, a.pos + a.T, threadIdx.x);
-    t.put(a.img + ((size_t)g * a.img_tiles + ti) * F::STAGE, threadIdx.x);
+    const int lane = threadIdx.x % OMH_WAVE, w = __builtin_amdgcn_readfirstlane(threadIdx.x / OMH_WAVE);
+    const size_t cache0 = ((size_t)a.seq * a.KV + g) * a.max_t * HD;
+    unsigned char *dst = a.img + ((size_t)g * a.img_tiles + ti) * F::TILE;
+    Flash3Frags<HD> k, v;
+    k.load_k(a.Kc + cache0, ti * F::KT, a.pos + a.T, w, lane);
+    v.load_v(a.Vc + cache0, ti * F::KT, a.pos + a.T, w, lane);
+    k.put(dst, w, lane);
+    v.put(dst + F::KB, w, lane);
+}
+
+// The products of the one-wave-per-SIMD form, with its output in accumulation
+// registers and everything else in vector registers for the whole sweep:
+// through the builtin the compiler puts all results in accumulation registers
+// and moves 128 of them to vector registers and back on every tile.  It does
+// not see what these instructions are, so their waits are here: two states
+// before each (an operand may just have been written by a VALU instruction,
+// a move between the register files among them; they pass while the product
+// before still runs), and acc_settle and vec_settle (a product's write lands
+// within 18 states) between the products and any other use of their results.
+__device__ __forceinline__ void acc_product(omh_v16f &c, const omh_v8bf &a, const omh_v8bf &b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void vec_product(omh_v16f &c, const omh_v8bf &a, const omh_v8bf &b) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, %0" : "+v"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void vec_product0(omh_v16f &c, const omh_v8bf &a, const omh_v8bf &b) {   // c = a b
+    asm volatile("s_nop 1\n\tv_mfma_f32_32x32x16_bf16 %0, %1, %2, 0" : "=&v"(c) : "v"(a), "v"(b));
+}
+__device__ __forceinline__ void vec_settle(omh_v16f &c, omh_v16f &d) { asm volatile("s_nop 15\n\ts_nop 3" : "+v"(c), "+v"(d)); }
+template <int N>
+__device__ __forceinline__ void acc_settle(omh_v16f (&c)[N]) {
+    asm volatile("s_nop 15\n\ts_nop 3" : "+a"(c[0]));
+#pragma unroll
+    for (int d = 1; d < N; d++) asm volatile("" : "+a"(c[d]));
+}
+// (no instruction: where control flow joins, a value whose only use is one
+// that wants accumulation registers stays in them)
+template <int N>
+__device__ __forceinline__ void acc_keep(omh_v16f (&c)[N]) {
+#pragma unroll
+    for (int d = 0; d < N; d++) asm volatile("" : "+a"(c[d]));
+}
+__device__ __forceinline__ void acc_scale(omh_v16f &c, float f) {
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+        float t, r;
+        asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(t) : "a"(c[i]));
+        t *= f;
+        asm volatile("v_accvgpr_write_b32 %0, %1" : "=a"(r) : "v"(t));
+        c[i] = r;
+    }
 }
 
 // IMG: each tile goes from its image (attn_tile_image_kernel) into LDS as
 // whole 1 KiB runs (buffer loads to LDS), with no conversion in the kernel.
 template <int HD, bool IMG>
-__global__ __launch_bounds__(8 * OMH_WAVE) __attribute__((amdgpu_waves_per_eu(2, 2)))
+__global__ __launch_bounds__(Flash3Shape<HD>::NW * OMH_WAVE)
+__attribute__((amdgpu_waves_per_eu(Flash3Shape<HD>::EU, Flash3Shape<HD>::EU)))
 void attn_flash3_kernel(const AttnArgs a) {
     using F = Flash3Shape<HD>;
-    constexpr int KT = F::KT, KLD = F::KLD, VLD = F::VLD, NS = F::NS, NJ = F::NJ;
+    constexpr int KT = F::KT, NS = F::NS, ND = F::ND, NW = F::NW;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem3[];
+    unsigned char *const Ks = smem3, *const Vs = smem3 + 2 * F::KB;
     const int H = a.H, KV = a.KV, grp = H / KV;
-    const int nunit = (a.T + 15) / 16 * grp, wpg = (nunit + 7) / 8;
-    const int g = blockIdx.x % KV, wi = wpg - 1 - (int)blockIdx.x / KV;
+    const int nunit = (a.T + 31) / 32 * grp, wpg = (nunit + NW - 1) / NW;
+    // the workgroups of one (kv head, key split) read the same tiles
+    const int gs = blockIdx.x % (KV * a.ns), g = gs % KV, sp = gs / KV;
+    const int wi = wpg - 1 - (int)(blockIdx.x / (KV * a.ns));   // the most keys first
     const int tid = threadIdx.x, lane = tid % OMH_WAVE;
     const int w = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
-    const int l16 = lane % 16, gq = lane / 16;
-    const bool own = 8 * wi + w < nunit;
-    const int u = min(8 * wi + w, nunit - 1);
+    const int l32 = lane % 32, g2 = lane / 32;
+    const bool own = NW * wi + w < nunit;
+    const int u = min(NW * wi + w, nunit - 1);
     const int tb = u / grp, h = g * grp + u % grp;
-    const int tq = 16 * tb + l16;                  // this lane's query token (may be past T: not written)
-    const int tlast = min(16 * (min(8 * wi + 7, nunit - 1) / grp) + 15, a.T - 1);
-    const int nkeys = a.pos + tlast + 1;
-    const int kmax = a.pos + tq;
+    const int tq = 32 * tb + l32;                  // this lane's query token (may be past T: not written)
+    const int tlast = min(32 * (min(NW * wi + NW - 1, nunit - 1) / grp) + 31, a.T - 1);
+    const int nkeys = a.pos + tlast + 1;           // keys the workgroup's last token sees
+    const int k0 = sp * a.kps, k1 = min(nkeys, k0 + a.kps);   // (kps is whole tiles)
+    if (k0 >= k1) return;                          // (the merge reads no such split)
+    const int kmax = a.pos + tq;                   // the last key this lane's token sees
 
-    // q as the B operand of S^T: dims 32 s + 8 gq .. +7 of token tq, hi and lo
+    // q as the B operand of S^T: dims 16 s + 8 g2 .. +7 of token tq, hi and lo
     omh_v8bf qh[NS], ql[NS];
     {
-        const float *qr = a.qb + ((size_t)min(tq, a.T - 1) * H + h) * HD + 8 * gq;
+        const float *qr = a.qb + ((size_t)min(tq, a.T - 1) * H + h) * HD + 8 * g2;
 #pragma unroll
         for (int s = 0; s < NS; s++) {
-            const float4 x0 = *reinterpret_cast<const float4 *>(qr + 32 * s);
-            const float4 x1 = *reinterpret_cast<const float4 *>(qr + 32 * s + 4);
+            const float4 x0 = *reinterpret_cast<const float4 *>(qr + 16 * s);
+            const float4 x1 = *reinterpret_cast<const float4 *>(qr + 16 * s + 4);
             const float v[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-#pragma unroll
-            for (int j = 0; j < 8; j++) {
-                qh[s][j] = (__bf16)v[j];
-                ql[s][j] = (__bf16)bf16_rest(v[j]);
-            }
+            bf16_split8(v, qh[s], ql[s]);
         }
     }
-    const size_t cache0 = ((size_t)a.seq * KV + g) * a.max_t;
-    const float *Kg = a.Kc + cache0 * HD, *Vg = a.Vc + cache0 * HD;
-    Flash3Tile<HD> tile;
-    // IMG: kv head g's tile images, F::STAGE bytes (whole 1 KiB runs) each
-    static_assert(F::STAGE % 1024 == 0, "an image tile is whole 1 KiB runs");
-    constexpr int NCH = F::STAGE / 1024;
+    const size_t cache0 = ((size_t)a.seq * KV + g) * a.max_t * HD;
+    const float *Kg = a.Kc + cache0, *Vg = a.Vc + cache0;
+    Flash3Frags<HD> fk, fv;
     const __amdgpu_buffer_rsrc_t irs =
-        omh_rsrc(IMG ? a.img + (size_t)g * a.img_tiles * F::STAGE : a.img, IMG ? a.img_tiles * F::STAGE : 0);
-    auto copy = [&](int kt, int stage) __attribute__((always_inline)) {
-        unsigned char *dst = smem3 + stage * F::STAGE;
-        const int src = kt / KT * F::STAGE;
+        omh_rsrc(IMG ? a.img + (size_t)g * a.img_tiles * F::TILE : a.img, IMG ? a.img_tiles * F::TILE : 0);
+    // IMG: half an image (K at 0, V at KB) of the tile at key kt into dst
+    auto copy = [&](int kt, int half, unsigned char *dst) __attribute__((always_inline)) {
+        const int src = kt / KT * F::TILE + half;
 #pragma unroll
-        for (int i = 0; i < (NCH + 7) / 8; i++) {
-            const int c = w + 8 * i;
-            if (c < NCH)
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void *)(dst + c * 1024),
-                                                         16, 16 * lane, src + c * 1024, 0, 0);
+        for (int i = 0; i < F::KB / 1024 / NW; i++) {
+            const int c = (w + NW * i) * 1024;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(irs, (__attribute__((address_space(3))) void *)(dst + c), 16,
+                                                     16 * lane, src + c, 0, 0);
         }
     };
-    auto load = [&](int kt) __attribute__((always_inline)) { tile.load(Kg, Vg, kt, nkeys, tid); };
-    auto put = [&](int stage) __attribute__((always_inline)) { tile.put(smem3 + stage * F::STAGE, tid); };
-
-    omh_v4f o[NJ];                                 // O^T: o[j][i] = O[token tq][dim 16 j + 4 gq + i]
-#pragma unroll
-    for (int j = 0; j < NJ; j++) o[j] = omh_v4f{0.f, 0.f, 0.f, 0.f};
-    float m = -INFINITY, l = 0.f;
-    if constexpr (IMG) {
-        copy(0, 0);
-        __builtin_amdgcn_s_waitcnt(0x0f70);     // vmcnt(0): this wave's copies have landed
-    } else {
-        load(0);
-        put(0);
-    }
-    __syncthreads();
-    for (int kt = 0, st = 0; kt < nkeys; kt += KT, st ^= 1) {
-        // (stage st ^ 1 was last read before the barrier that ended the previous step)
-        if (kt + KT < nkeys) {
-            if constexpr (IMG) copy(kt + KT, st ^ 1);
-            else load(kt + KT);
-        }
-        const unsigned char *sb = smem3 + st * F::STAGE;
-        const unsigned char *Kh = sb, *Kl = sb + F::KPL, *Vh = sb + 2 * F::KPL, *Vl = Vh + F::VPL;
-        // S^T for keys kt + 16 n + 4 gq + i (register i of sc[n]), query row tq
-        omh_v4f sc[KT / 16];
-#pragma unroll
-        for (int n = 0; n < KT / 16; n++) {
-            sc[n] = omh_v4f{0.f, 0.f, 0.f, 0.f};
-            const size_t ro = (size_t)(16 * n + l16) * KLD + 16 * gq;
-#pragma unroll
-            for (int s = 0; s < NS; s++) {
-                const omh_v8bf kh = *reinterpret_cast<const omh_v8bf *>(Kh + ro + 64 * s);
-                const omh_v8bf kl = *reinterpret_cast<const omh_v8bf *>(Kl + ro + 64 * s);
-                sc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, qh[s], sc[n], 0, 0, 0);
-                sc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kh, ql[s], sc[n], 0, 0, 0);
-                sc[n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kl, qh[s], sc[n], 0, 0, 0);
-            }
-        }
-        // scores * hd^-1/2, causal mask, online softmax (qwen.c:410-414)
-        float mx = -INFINITY;
-#pragma unroll
-        for (int n = 0; n < KT / 16; n++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const int key = kt + 16 * n + 4 * gq + i;
-                sc[n][i] = key <= kmax ? sc[n][i] * a.scale : -INFINITY;
-                mx = fmaxf(mx, sc[n][i]);
-            }
-        mx = omh_swap32_max(omh_swap16_max(mx));
-        const float mn = fmaxf(m, mx);             // finite: key 0 is in every token's first tile
-        // e^(s - mn) as 2^((s - mn) log2 e) on the hardware exp2 (a masked
-        // score, -inf, gives 0; the first tile's corr, 2^-inf, 0)
-        const float corr = __builtin_amdgcn_exp2f((m - mn) * 1.4426950408889634f);
-        float ps = 0.f;
-        omh_v8bf ph, pl;                           // P^T as the B operand: j = 4 n + i
-#pragma unroll
-        for (int n = 0; n < KT / 16; n++)
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float pv = __builtin_amdgcn_exp2f((sc[n][i] - mn) * 1.4426950408889634f);
-                ps += pv;
-                ph[4 * n + i] = (__bf16)pv;
-                pl[4 * n + i] = (__bf16)bf16_rest(pv);
-            }
-        ps = omh_swap32_sum(omh_swap16_sum(ps));
-        l = fmaf(l, corr, ps);
-        m = mn;
-        // O^T = corr O^T + V^T P^T (qwen.c:415-419); the rescale only when a
-        // row's max moved (corr = 1 otherwise)
-        if (__builtin_amdgcn_ballot_w64(corr != 1.f))
-#pragma unroll
-            for (int j = 0; j < NJ; j++) o[j] = o[j] * corr;
-#pragma unroll
-        for (int j = 0; j < NJ; j++) {
-            const size_t ro = (size_t)(16 * j + l16) * VLD + 16 * gq;
-            const omh_v8bf vh = *reinterpret_cast<const omh_v8bf *>(Vh + ro);
-            const omh_v8bf vl = *reinterpret_cast<const omh_v8bf *>(Vl + ro);
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, ph, o[j], 0, 0, 0);
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vh, pl, o[j], 0, 0, 0);
-            o[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vl, ph, o[j], 0, 0, 0);
-        }
-        if constexpr (IMG) __builtin_amdgcn_s_waitcnt(0x0f70);
-        else if (kt + KT < nkeys) put(st ^ 1);
+    // fetch: request K of tile kt into K stage st (reg form: into registers,
+    // land() stores them once the stage is free)
+    auto fetch_k = [&](int kt, int st) __attribute__((always_inline)) {
+        if constexpr (IMG) copy(kt, 0, Ks + st * F::KB);
+        else fk.load_k(Kg, kt, nkeys, w, lane);
+    };
+    auto fetch_v = [&](int kt, int st) __attribute__((always_inline)) {
+        if constexpr (IMG) copy(kt, F::KB, Vs + st * F::VB);
+        else fv.load_v(Vg, kt, nkeys, w, lane);
+    };
+    auto land_k = [&](int st) __attribute__((always_inline)) {
+        if constexpr (!IMG) fk.put(Ks + st * F::KB, w, lane);
+    };
+    auto land_v = [&](int st) __attribute__((always_inline)) {
+        if constexpr (!IMG) fv.put(Vs + st * F::VB, w, lane);
+    };
+    auto arrive = [&]() __attribute__((always_inline)) {
+        if constexpr (IMG) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies have landed
         __syncthreads();
-    }
-    // normalise and gate (qwen.c:420-421)
-    if (!own || tq >= a.T) return;
-    const float il = 1.f / l;
-    const float *gate = a.qkv + (size_t)tq * a.ld_qkv + (size_t)h * 2 * HD + HD + 4 * gq;
-    float *dst = a.ctx + ((size_t)tq * H + h) * HD + 4 * gq;
+    };
+
+    omh_v16f o[ND];                                // O^T: o[d][i] = O[token tq][dim 32 d + 8 (i / 4) + 4 g2 + i % 4]
 #pragma unroll
-    for (int j = 0; j < NJ; j++) {
-        const float4 gv = *reinterpret_cast<const float4 *>(gate + 16 * j);
-        float4 r;
-        r.x = o[j][0] * il * omh_sigmoid(gv.x);
-        r.y = o[j][1] * il * omh_sigmoid(gv.y);
-        r.z = o[j][2] * il * omh_sigmoid(gv.z);
-        r.w = o[j][3] * il * omh_sigmoid(gv.w);
-        *reinterpret_cast<float4 *>(dst + 16 * j) = r;
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int i = 0; i < 16; i++) o[d][i] = 0.f;
+    float m = -INFINITY, l = 0.f;                  // reference of the raw scores (q.k), sum of the weights
+    const float sl2 = a.scale * 1.4426950408889634f;   // hd^-1/2 log2 e (qwen.c:410-414)
+
+    // The work of one iteration, in a fixed order (sched_barriers between
+    // the steps: left to itself the compiler reads each fragment right
+    // before its products, and a lone wave then waits out every LDS read).
+    // Step i of a block takes fragment pairs (hi, lo) 2 i and 2 i + 1 through
+    // their three products each, on two accumulators in turn (a product on
+    // the accumulator of the one right before it waits twice as long),
+    // requests pairs 2 i + AHEAD and the next, and does a piece of the softmax.
+    constexpr int AHEAD = 4;
+    omh_v8bf rh[AHEAD], rl[AHEAD];                 // the pairs in flight
+    const int l16 = 16 * lane;
+    omh_v16f sc, sd;                               // S^T of a tile: even and odd steps' sums
+    omh_v8bf ph[2], pl[2];                         // P^T as the B operand of 16-key step u
+    omh_v4u32 nh[2], nl[2];                        // the next tile's
+    float mx, ps, ref, corr = 1.f;
+    auto ask = [&](const unsigned char *base, auto pair) __attribute__((always_inline)) {
+        constexpr int P = decltype(pair)::value;
+        rh[P % AHEAD] = *reinterpret_cast<const omh_v8bf *>(base + l16 + 2048 * P);
+        rl[P % AHEAD] = *reinterpret_cast<const omh_v8bf *>(base + l16 + 2048 * P + 1024);
+    };
+    auto product = [&](omh_v16f &c, const omh_v8bf &x, const omh_v8bf &y) __attribute__((always_inline)) {
+        if constexpr (F::EU == 1) vec_product(c, x, y);
+        else c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+    };
+    auto product0 = [&](omh_v16f &c, const omh_v8bf &x, const omh_v8bf &y) __attribute__((always_inline)) {
+        if constexpr (F::EU == 1) vec_product0(c, x, y);
+        else {
+            const omh_v16f zero = {};
+            c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, zero, 0, 0, 0);
+        }
+    };
+    auto add_product = [&](omh_v16f &c, const omh_v8bf &x, const omh_v8bf &y) __attribute__((always_inline)) {
+        if constexpr (F::EU == 1) acc_product(c, x, y);
+        else c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(x, y, c, 0, 0, 0);
+    };
+    // step s of the scores of the K tile at kb; with then_v the last steps
+    // ask for the first V pairs at vb
+    auto score_step = [&](auto step, const unsigned char *kb, auto then_v, const unsigned char *vb) __attribute__((always_inline)) {
+        constexpr int S = 2 * decltype(step)::value, R = S % AHEAD;
+        const omh_v8bf h0 = rh[R], l0 = rl[R], h1 = rh[R + 1], l1 = rl[R + 1];
+        if constexpr (S == 0) {
+            product0(sc, l0, qh[S]);
+            product0(sd, l1, qh[S + 1]);
+        } else {
+            product(sc, l0, qh[S]);
+            product(sd, l1, qh[S + 1]);
+        }
+        product(sc, h0, ql[S]);
+        product(sd, h1, ql[S + 1]);
+        product(sc, h0, qh[S]);
+        product(sd, h1, qh[S + 1]);
+        if constexpr (S + AHEAD < NS) {
+            ask(kb, std::integral_constant<int, S + AHEAD>{});
+            ask(kb, std::integral_constant<int, S + AHEAD + 1>{});
+        } else if constexpr (decltype(then_v)::value) {
+            ask(vb, std::integral_constant<int, S + AHEAD - NS>{});
+            ask(vb, std::integral_constant<int, S + AHEAD + 1 - NS>{});
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // Causal mask and online softmax of the tile at key kt (qwen.c:410-414),
+    // in pieces 0 .. NP - 1.  The reference moves only where a score exceeds
+    // it by 2^kSlack (the weights then stay below 2^kSlack, well inside fp32
+    // and its bf16 pairs), so o is hardly ever rescaled: with the running max
+    // itself some of a wave's 32 rows move on most of a prompt's tiles.
+    constexpr int NP = 14;
+    constexpr float kSlack = 8.f;
+    auto soften = [&](auto piece, int kt) __attribute__((always_inline)) {
+        constexpr int P = decltype(piece)::value;
+        if constexpr (P == 0 && F::EU == 1) {
+            vec_settle(sc, sd);
+        }
+        if constexpr (P < 4) {
+            const int left = kmax - kt - 4 * g2;   // key 8 (i / 4) + i % 4 of this lane is visible up to here
+#pragma unroll
+            for (int i = 4 * P; i < 4 * P + 4; i++) sc[i] = 8 * (i / 4) + i % 4 <= left ? sc[i] + sd[i] : -INFINITY;
+            const float m4 = fmaxf(fmaxf(sc[4 * P], sc[4 * P + 1]), fmaxf(sc[4 * P + 2], sc[4 * P + 3]));
+            mx = P == 0 ? m4 : fmaxf(mx, m4);
+        } else if constexpr (P == 4) {
+            mx = omh_swap32_max(mx);
+            const bool none = m == -INFINITY, moves = none | ((mx - m) * sl2 > kSlack);
+            const float shrink = __builtin_amdgcn_exp2f((m - mx) * sl2);
+            corr = (moves & !none) ? shrink : 1.f;
+            m = moves ? mx : m;
+            // (a split may begin past some of its tokens' keys: nothing seen
+            // yet, and every weight 2^-inf = 0 against any finite reference)
+            ref = m == -INFINITY ? 0.f : m * sl2;
+            ps = 0.f;
+        } else if constexpr (P < 13) {
+            constexpr int E = 2 * (P - 5);
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(sc[E], sl2, -ref));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(sc[E + 1], sl2, -ref));
+            ps += p0;
+            ps += p1;
+            uint32_t hi, lo;
+            bf16_split2(p0, p1, hi, lo);
+            nh[E / 8][E % 8 / 2] = hi;
+            nl[E / 8][E % 8 / 2] = lo;
+            // (formed here, not behind the rescale's branch)
+            if constexpr (P == 8 || P == 12) asm volatile("" : "+v"(nh[P / 4 - 2]), "+v"(nl[P / 4 - 2]));
+        } else {
+            l = fmaf(l, corr, omh_swap32_sum(ps));
+        }
+    };
+    auto turn = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < 2; u++) {
+            ph[u] = __builtin_bit_cast(omh_v8bf, nh[u]);
+            pl[u] = __builtin_bit_cast(omh_v8bf, nl[u]);
+        }
+    };
+    // step i of O^T += V^T P^T for the V tile at vb: output tiles 2 (i / 2)
+    // and the next, 16-key step i % 2
+    auto weigh_step = [&](auto step, const unsigned char *vb) __attribute__((always_inline)) {
+        constexpr int I = decltype(step)::value, d = 2 * (I / 2), u = I % 2, R = 2 * I % AHEAD;
+        const omh_v8bf h0 = rh[R], l0 = rl[R], h1 = rh[R + 1], l1 = rl[R + 1];
+        add_product(o[d], l0, ph[u]);
+        add_product(o[d + 1], l1, ph[u]);
+        add_product(o[d], h0, pl[u]);
+        add_product(o[d + 1], h1, pl[u]);
+        add_product(o[d], h0, ph[u]);
+        add_product(o[d + 1], h1, ph[u]);
+        if constexpr (2 * I + AHEAD < 2 * ND) {
+            ask(vb, std::integral_constant<int, 2 * I + AHEAD>{});
+            ask(vb, std::integral_constant<int, 2 * I + AHEAD + 1>{});
+        }
+    };
+    // O^T = corr O^T (qwen.c:415-419), where some row's reference moved
+    auto rescale = [&]() __attribute__((always_inline)) {
+        if (!__builtin_amdgcn_ballot_w64(corr != 1.f)) return;
+        if constexpr (F::EU == 1) {
+            acc_settle(o);
+#pragma unroll
+            for (int d = 0; d < ND; d++) acc_scale(o[d], corr);
+            acc_settle(o);
+        } else {
+#pragma unroll
+            for (int d = 0; d < ND; d++) o[d] = o[d] * corr;
+        }
+    };
+    fetch_k(k0, 0);
+    fetch_v(k0, 0);
+    land_k(0);
+    if (k0 + KT < k1) fetch_k(k0 + KT, 1);
+    land_v(0);
+    if (k0 + KT < k1) land_k(1);
+    arrive();
+    static_assert(NS % AHEAD == 0 && NS == 2 * ND && AHEAD % 2 == 0, "pairs in flight");
+    constexpr int STEPS = NS / 2;
+    omh_static_for<AHEAD>([&](auto i) { ask(Ks, i); });
+    omh_static_for<STEPS>([&](auto i) { score_step(i, Ks, std::false_type{}, nullptr); });
+    omh_static_for<NP>([&](auto i) { soften(i, k0); });   // (o is still zero: nothing to rescale)
+    turn();
+    if constexpr (F::EU == 1) acc_keep(o);
+    int kt = k0, st = 0;
+    for (; kt + KT < k1; kt += KT, st ^= 1) {
+        // K stage st held tile kt, whose scores every wave has formed, and V
+        // stage st ^ 1 the tile before it, which every wave has added
+        if constexpr (F::EU == 1) acc_keep(o);
+        __syncthreads();
+        const unsigned char *kb = Ks + (st ^ 1) * F::KB, *vb = Vs + st * F::VB;
+        omh_static_for<AHEAD>([&](auto i) { ask(kb, i); });
+        __builtin_amdgcn_sched_barrier(0);
+        if (kt + 2 * KT < k1) fetch_k(kt + 2 * KT, st);
+        fetch_v(kt + KT, st ^ 1);
+        __builtin_amdgcn_sched_barrier(0);
+        omh_static_for<STEPS>([&](auto i) { score_step(i, kb, std::true_type{}, vb); });
+        omh_static_for<STEPS>([&](auto i) {
+            constexpr int I = decltype(i)::value, PER = (NP + STEPS - 2) / (STEPS - 1);   // (the scores land during step 0)
+            weigh_step(i, vb);
+            if constexpr (I > 0)
+                omh_static_for<PER>([&](auto j) {
+                    constexpr int P = PER * (I - 1) + decltype(j)::value;
+                    if constexpr (P < NP) soften(std::integral_constant<int, P>{}, kt + KT);
+                });
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        turn();
+        rescale();
+        if constexpr (F::EU == 1) acc_keep(o);
+        if (kt + 2 * KT < k1) land_k(st);
+        land_v(st ^ 1);
+        // this wave's copies (IMG: vmcnt(0)) or LDS stores (lgkmcnt(0): this
+        // compiler leaves the wait for stores before a loop's back edge out
+        // of the barrier at its head) have landed
+        __builtin_amdgcn_s_waitcnt(IMG ? 0x0f70 : 0xc07f);
     }
+    if constexpr (F::EU == 1) acc_keep(o);
+    __syncthreads();
+    const unsigned char *vb = Vs + st * F::VB;
+    omh_static_for<AHEAD>([&](auto i) { ask(vb, i); });
+    omh_static_for<STEPS>([&](auto i) { weigh_step(i, vb); });
+    if constexpr (F::EU == 1) acc_settle(o);
+
+    if (!own || tq >= a.T) return;
+    if (a.ns > 1) {
+        // unnormalised partial of split sp (the reference in the scaled scores' units)
+        const size_t pi = ((size_t)tq * H + h) * a.ns + sp;
+        float *dst = a.po + pi * HD + 4 * g2;
+#pragma unroll
+        for (int d = 0; d < ND; d++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                *reinterpret_cast<float4 *>(dst + 32 * d + 8 * k) =
+                    make_float4(o[d][4 * k], o[d][4 * k + 1], o[d][4 * k + 2], o[d][4 * k + 3]);
+        if (g2 == 0) {
+            a.pml[2 * pi] = m * a.scale;
+            a.pml[2 * pi + 1] = l;
+        }
+        return;
+    }
+    // normalise and gate (qwen.c:420-421); the hardware sigmoid, because 128
+    // of the library's are 4000 instructions: 7 us at the end of a workgroup
+    const float il = 1.f / l;
+    const float *gate = a.qkv + (size_t)tq * a.ld_qkv + (size_t)h * 2 * HD + HD + 4 * g2;
+    float *dst = a.ctx + ((size_t)tq * H + h) * HD + 4 * g2;
+#pragma unroll
+    for (int d = 0; d < ND; d++)
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const float4 gv = *reinterpret_cast<const float4 *>(gate + 32 * d + 8 * k);
+            float4 r;
+            r.x = o[d][4 * k] * il * omh_sigmoid_fast(gv.x);
+            r.y = o[d][4 * k + 1] * il * omh_sigmoid_fast(gv.y);
+            r.z = o[d][4 * k + 2] * il * omh_sigmoid_fast(gv.z);
+            r.w = o[d][4 * k + 3] * il * omh_sigmoid_fast(gv.w);
+            *reinterpret_cast<float4 *>(dst + 32 * d + 8 * k) = r;
+        }
+}
+
+// The flash kernel's splits merged, normalised and gated: a wave per (token,
+// head) row (two at HD = 128), lane = 4 columns.  Token t has a partial in
+// every split that begins at or before its position.
+template <int HD>
+__global__ __launch_bounds__(256) void attn_flash_merge_kernel(const AttnArgs a) {
+    constexpr int LR = HD / 4;                     // lanes per row
+    const size_t th = (size_t)blockIdx.x * (256 / LR) + threadIdx.x / LR;
+    if (th >= (size_t)a.T * a.H) return;
+    const int c = 4 * (threadIdx.x % LR), t = (int)(th / a.H), h = (int)(th % a.H);
+    const int nl = (a.pos + t) / a.kps + 1;        // live splits
+    const float *ml = a.pml + 2 * th * a.ns, *po = a.po + th * a.ns * HD + c;
+    float M = -INFINITY;
+    for (int s = 0; s < nl; s++) M = fmaxf(M, ml[2 * s]);
+    float L = 0.f;
+    float4 o = f4_zero();
+#pragma unroll 4
+    for (int s = 0; s < nl; s++) {
+        const float f = expf(ml[2 * s] - M);
+        L = fmaf(ml[2 * s + 1], f, L);
+        o = f4_fma(*reinterpret_cast<const float4 *>(po + (size_t)s * HD), f, o);
+    }
+    const float il = 1.f / L;
+    const float4 gv = *reinterpret_cast<const float4 *>(a.qkv + (size_t)t * a.ld_qkv + (size_t)h * 2 * HD + HD + c);
+    float4 r;
+    r.x = o.x * il * omh_sigmoid(gv.x);
+    r.y = o.y * il * omh_sigmoid(gv.y);
+    r.z = o.z * il * omh_sigmoid(gv.z);
+    r.w = o.w * il * omh_sigmoid(gv.w);
+    *reinterpret_cast<float4 *>(a.ctx + th * HD + c) = r;
 }
 
 // One workgroup per (token, head, 64 columns): the CW waves take every
@@ -1136,31 +1386,39 @@ hipError_t launch_attn_d(const AttnArgs &a, hipStream_t st) {
     if (!fuse) hipLaunchKernelGGL((attn_prep_kernel<HD>), dim3((unsigned)a.T), dim3(kPrepWaves * OMH_WAVE), 0, st, a);
     if constexpr (HD >= 128) {
         if (attn_uses_flash(a.T, HD)) {
-            const int wpg = ((a.T + 15) / 16 * (a.H / a.KV) + 7) / 8;
-            const dim3 grid((unsigned)(a.KV * wpg)), blk(8 * OMH_WAVE);
             if (flash_fp32()) {
+                const int wpg = ((a.T + 15) / 16 * (a.H / a.KV) + 7) / 8;
                 static const bool ok = hipFuncSetAttribute((const void *)attn_flash_kernel<HD>,
                                                            hipFuncAttributeMaxDynamicSharedMemorySize,
                                                            (int)FlashShape<HD>::LDS) == hipSuccess;
                 if (!ok) return hipErrorInvalidValue;
-                hipLaunchKernelGGL((attn_flash_kernel<HD>), grid, blk, FlashShape<HD>::LDS, st, a);
+                hipLaunchKernelGGL((attn_flash_kernel<HD>), dim3((unsigned)(a.KV * wpg)), dim3(8 * OMH_WAVE),
+                                   FlashShape<HD>::LDS, st, a);
+                return hipGetLastError();
+            }
+            using F = Flash3Shape<HD>;
+            const int wpg = ((a.T + 31) / 32 * (a.H / a.KV) + F::NW - 1) / F::NW;
+            if (a.kps % F::KT != 0) return hipErrorInvalidValue;
+            static const bool ok =
+                hipFuncSetAttribute((const void *)attn_flash3_kernel<HD, false>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)F::LDS) == hipSuccess &&
+                hipFuncSetAttribute((const void *)attn_flash3_kernel<HD, true>,
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)F::LDS) == hipSuccess;
+            if (!ok) return hipErrorInvalidValue;
+            const dim3 grid((unsigned)(a.KV * a.ns * wpg)), blk(F::NW * OMH_WAVE);
+            if (a.img) {
+                // the images of every tile of keys 0 .. pos + T - 1, then the kernel copying them
+                const long tiles = ((long)a.pos + a.T + F::KT - 1) / F::KT;
+                if (a.img_tiles != tiles || (size_t)tiles * F::TILE > (size_t)INT32_MAX) return hipErrorInvalidValue;
+                hipLaunchKernelGGL((attn_tile_image_kernel<HD>), dim3((unsigned)(a.KV * tiles)), blk, 0, st, a);
+                hipLaunchKernelGGL((attn_flash3_kernel<HD, true>), grid, blk, F::LDS, st, a);
             } else {
-                static const bool ok =
-                    hipFuncSetAttribute((const void *)attn_flash3_kernel<HD, false>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)Flash3Shape<HD>::LDS) == hipSuccess &&
-                    hipFuncSetAttribute((const void *)attn_flash3_kernel<HD, true>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)Flash3Shape<HD>::LDS) == hipSuccess;
-                if (!ok) return hipErrorInvalidValue;
-                if (a.img) {
-                    // the images of every tile of keys 0 .. pos + T - 1, then the kernel copying them
-                    const long tiles = ((long)a.pos + a.T + Flash3Shape<HD>::KT - 1) / Flash3Shape<HD>::KT;
-                    if (a.img_tiles != tiles || (size_t)tiles * Flash3Shape<HD>::STAGE > (size_t)INT32_MAX)
-                        return hipErrorInvalidValue;
-                    hipLaunchKernelGGL((attn_tile_image_kernel<HD>), dim3((unsigned)(a.KV * tiles)), blk, 0, st, a);
-                    hipLaunchKernelGGL((attn_flash3_kernel<HD, true>), grid, blk, Flash3Shape<HD>::LDS, st, a);
-                } else {
-                    hipLaunchKernelGGL((attn_flash3_kernel<HD, false>), grid, blk, Flash3Shape<HD>::LDS, st, a);
-                }
+                hipLaunchKernelGGL((attn_flash3_kernel<HD, false>), grid, blk, F::LDS, st, a);
+            }
+            if (a.ns > 1) {
+                constexpr int rows = 256 / (HD / 4);
+                hipLaunchKernelGGL((attn_flash_merge_kernel<HD>), dim3((unsigned)(((size_t)a.T * a.H + rows - 1) / rows)),
+                                   dim3(256), 0, st, a);
             }
             return hipGetLastError();
         }
@@ -1211,9 +1469,9 @@ size_t flash_image_bytes_d(int KV, int pos, int T, int *tiles) {
     const size_t n = ((size_t)pos + T + F::KT - 1) / F::KT;
     // one kv head's images are addressed with 32-bit buffer offsets: longer
     // steps stage their tiles in the kernel
-    if (n * F::STAGE > (size_t)INT32_MAX) return 0;
+    if (n * F::TILE > (size_t)INT32_MAX) return 0;
     *tiles = (int)n;
-    return (size_t)KV * n * F::STAGE;
+    return (size_t)KV * n * F::TILE;
 }
 
 size_t attn_flash_image_bytes(int hd, int KV, int pos, int T, int *tiles) {
@@ -1235,6 +1493,40 @@ void attn_plan(int pos, int T, int KV, int &ns, int &kps) {
     k = (k + 63) / 64 * 64;
     kps = (int)k;
     ns = (int)((nmax + k - 1) / k);
+}
+
+// Key splits of a prompt step on the flash kernel, by an estimate of its time
+// in 32-key tiles of one workgroup (about 1.6 us): the workgroups of a split
+// sweep their tiles with kEnds tiles' worth of prologue and epilogue, one per
+// CU at a time (two at head width 128); their partials are written and read
+// once at about 4 TB/s.  One split where the unsplit workgroups fill the chip.
+void attn_flash_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
+    constexpr int KT = 32, NW = 4, kMaxSplits = 64;
+    constexpr double kEnds = 3, kBytesPerTile = 6.4e6;
+    const long nt = ((long)pos + T + KT - 1) / KT;
+    const long wpg = ((long)(T + 31) / 32 * (H / KV) + NW - 1) / NW;
+    const double avg = 0.5 * ((double)nt + (double)(pos / KT + 1));   // tiles of a workgroup, unsplit
+    const double slots = hd > 128 ? 256 : 512;
+    double best = 0;
+    ns = 1;
+    kps = (int)(nt * KT);
+    if (flash_fp32()) return;
+    for (int s = 1; s <= kMaxSplits && s <= nt; s++) {
+        const long tps = (nt + s - 1) / s;
+        if ((nt + tps - 1) / tps != s) continue;              // the same split as an earlier s
+        const double per = s == 1 ? 1 : std::min((double)s, avg / tps + 0.5);   // live splits of a workgroup
+        const double units = (double)KV * wpg * per, sum = (double)KV * wpg * avg;
+        double cost = tps + kEnds;
+        if (units > slots)
+            cost = std::max(std::ceil(units / slots) * (sum / units + kEnds),
+                            (sum + kEnds * units) / slots + 0.25 * (tps + kEnds));
+        if (s > 1) cost += 2 + (double)T * H * per * hd * 8 / kBytesPerTile;
+        if (s == 1 || cost < best) {
+            best = cost;
+            ns = s;
+            kps = (int)(tps * KT);
+        }
+    }
 }
 
 hipError_t launch_attn(const AttnArgs &a, int hd, hipStream_t st) {

@@ -52,15 +52,6 @@ __device__ __forceinline__ void wait_vmcnt(int n) {
     if constexpr (N > 0) wait_vmcnt<N - 1>(n);
 }
 
-// f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
-template <int N, int I = 0, typename F>
-__device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
-
 // Weight fragment: 16 consecutive weights of one row, as loaded (int8 or
 // fp32) and as fp32.
 template <bool Q8>
@@ -683,7 +674,7 @@ void proj_q8_bf16x3_kernel(const ProjArgs p) {
 
     // the prologue issues x then w per block, as the loop does, so the wait
     // counts are the same on entry and on the back edge
-    static_for<PF>([&](auto sc) __attribute__((always_inline)) {
+    omh_static_for<PF>([&](auto sc) __attribute__((always_inline)) {
         constexpr int s = decltype(sc)::value;
         if constexpr (s < XD) x_load(s, std::integral_constant<int, s>{});
         w_load(s, sc);
@@ -692,7 +683,7 @@ void proj_q8_bf16x3_kernel(const ProjArgs p) {
     x_load(XD, std::integral_constant<int, 0>{});
     // PF divides nb
     auto step = [&](int b0) __attribute__((always_inline)) {
-        static_for<PF>([&](auto sc) __attribute__((always_inline)) {
+        omh_static_for<PF>([&](auto sc) __attribute__((always_inline)) {
             constexpr int s = decltype(sc)::value;
             const int b = b0 + s;
             const int buf = b & 1;
@@ -941,12 +932,12 @@ void proj_q8_wave_kernel(const ProjArgs p, int nb, const F32Part f) {
             if (b0 + u / 2 + WD >= 0) w_load(b0 + u / 2 + WD, std::integral_constant<int, u / 2>{});
     };
     // prologue: the previous iteration's loads (b0 = -WD), without products
-    static_for<2 * WD>([&](auto uc) __attribute__((always_inline)) { loads_at(-WD, uc, std::false_type{}); });
+    omh_static_for<2 * WD>([&](auto uc) __attribute__((always_inline)) { loads_at(-WD, uc, std::false_type{}); });
 #pragma unroll 1
     for (int b0 = 0; b0 < nb; b0 += WD) {
         // (the scheduler would otherwise sink each prefetch next to its
         // use, where its wait drains everything in flight)
-        static_for<2 * WD>([&](auto uc) __attribute__((always_inline)) { loads_at(b0, uc, std::true_type{}); });
+        omh_static_for<2 * WD>([&](auto uc) __attribute__((always_inline)) { loads_at(b0, uc, std::true_type{}); });
     }
 
     // the workgroup's 4 k-subslices, in wave order; wave w then finishes
@@ -1811,7 +1802,7 @@ void proj_i8_stream_kernel(const ProjArgs p, const F32Part f) {
     // the first x pieces, then all of the wave's weights block by block,
     // then x XR - 1 pieces ahead of the products.  Loads retire in issue
     // order, so the products of block b wait only for the weights up to b.
-    static_for<XR - 1>([&](auto qc) __attribute__((always_inline)) {
+    omh_static_for<XR - 1>([&](auto qc) __attribute__((always_inline)) {
         if constexpr (decltype(qc)::value < NQ) x_load(qc);
     });
 #pragma unroll
@@ -1823,7 +1814,7 @@ void proj_i8_stream_kernel(const ProjArgs p, const F32Part f) {
             for (int h = 0; h < 2; h++) wq[b][rt][h] = __builtin_nontemporal_load(reinterpret_cast<const v4i *>(src + 64 * h));
         }
     __builtin_amdgcn_sched_barrier(0);
-    static_for<NQ>([&](auto qc) __attribute__((always_inline)) {
+    omh_static_for<NQ>([&](auto qc) __attribute__((always_inline)) {
         constexpr int q = decltype(qc)::value, b = q / NT, nt = q % NT, sl = q % XR;
         if constexpr (q + XR - 1 < NQ) x_load(std::integral_constant<int, q + XR - 1>{});
         __builtin_amdgcn_sched_barrier(0);
@@ -2032,7 +2023,7 @@ void proj_i8_dq_kernel(const ProjArgs p, const F32Part f) {
         // block: the epilogue would wait for those loads)
         if (NBC == 0 || b + kDqX < NB) x_load(b + kDqX, slot_c);
     };
-    static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { x_load(decltype(sc)::value, sc); });
+    omh_static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { x_load(decltype(sc)::value, sc); });
     w_read(0, std::integral_constant<int, 0>{});
     if constexpr (NBC > 0) {
         // (straight-line code: the x ring's waits count exactly the loads
@@ -2040,11 +2031,11 @@ void proj_i8_dq_kernel(const ProjArgs p, const F32Part f) {
         // back edge)
 #pragma unroll
         for (int b = 0; b < NBC; b += kDqX)
-            static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { block(b + decltype(sc)::value, sc); });
+            omh_static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { block(b + decltype(sc)::value, sc); });
     } else {
 #pragma unroll 1
         for (int b = 0; b < NB; b += kDqX)
-            static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { block(b + decltype(sc)::value, sc); });
+            omh_static_for<kDqX>([&](auto sc) __attribute__((always_inline)) { block(b + decltype(sc)::value, sc); });
     }
 
     // lane holds rows 4gq .. 4gq+3 of row tile rt for token l16 of token tile w

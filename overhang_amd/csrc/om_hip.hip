@@ -458,12 +458,14 @@ int attn_forward(int li, int seq, int pos, int T, const float *x, float *out, hi
     if (!x || !out || !aligned16(x) || !aligned16(out)) return fail(OMH_ERR_ARG, "attn: x/out must be 16-byte aligned");
     const int D = d.hidden, hd = d.head_dim, H = d.n_heads;
     int ns = 0, kps = 0;
-    attn_plan(pos, T, d.n_kv, ns, kps);
+    const bool flash = attn_uses_flash(T, hd);
+    if (flash) attn_flash_plan(pos, T, H, d.n_kv, hd, ns, kps);
+    else attn_plan(pos, T, d.n_kv, ns, kps);
     const size_t nth = (size_t)T * H;
     if (int rc = ensure(g_arow, (size_t)T * A.rows * sizeof(float))) return rc;
     if (int rc = ensure(g_aqb, nth * hd * sizeof(float))) return rc;
     if (int rc = ensure(g_actx, nth * hd * sizeof(float))) return rc;
-    if (!attn_uses_flash(T, hd)) {                    // (the flash kernel keeps no split partials)
+    if (!flash || ns > 1) {                           // (an unsplit flash step keeps no partials)
         if (int rc = ensure(g_apo, nth * ns * hd * sizeof(float))) return rc;
         if (int rc = ensure(g_apml, nth * ns * 2 * sizeof(float))) return rc;
     }

@@ -213,9 +213,9 @@ struct AttnArgs {
     float *po, *pml;                   // [T][H][ns][hd] partial outputs, [T][H][ns][2] running max and sum
     float *ctx;                        // [T][H * hd] gated attention output
     int seq, pos, T, H, KV, rot, max_t;
-    int ns, kps;                       // key splits and keys per split (attn_plan)
+    int ns, kps;                       // key splits and keys per split (attn_plan, attn_flash_plan)
     float eps, scale;                  // RMSNorm eps, hd^-1/2
-    unsigned char *img;                // or null: the bf16 x 3 flash kernel's tile images [KV][img_tiles][stage]
+    unsigned char *img;                // or null: the bf16 x 3 flash kernel's tile images [KV][img_tiles][tile]
     int img_tiles;                     //   (attn_flash_image_bytes), made in the same call from the cache
 };
 bool attn_supported(int hd, int H, int KV, int rot);
@@ -227,6 +227,8 @@ size_t attn_flash_image_bytes(int hd, int KV, int pos, int T, int *tiles);
 bool attn_uses_flash(int T, int hd);
 // splits for pos + T visible keys: ns * KV * T >= 256 workgroups where the keys allow
 void attn_plan(int pos, int T, int KV, int &ns, int &kps);
+// the same for a prompt step on the flash kernel (kps whole 32-key tiles; ns = 1: no partials)
+void attn_flash_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps);
 hipError_t launch_attn(const AttnArgs &a, int hd, hipStream_t st);
 
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported shape.

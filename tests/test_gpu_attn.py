@@ -329,3 +329,31 @@ def test_decode_prep_in_split_kernel_matches_prep_launch(shape, monkeypatch):
             L.free()
     for a, b, nm in zip(outs["1"], outs["0"], ("out", "K cache", "V cache")):
         np.testing.assert_array_equal(a, b, err_msg=f"{shape} fused prep vs prep launch: {nm}")
+
+
+@pytest.mark.parametrize("shape,pos,T", [(Q35B_ATTN, 1500, 64), (Q35B_ATTN, 995, 97), (Q35B_ATTN, 31, 255),
+                                         (Q35B_ATTN, 1401, 256), ((512, 16, 1, 128, 128), 2040, 65),
+                                         ((1024, 4, 4, 256, 256), 640, 300)],
+                         ids=["pos1500-T64", "pos995-T97", "pos31-T255", "pos1401-T256", "hd128-pos2040-T65",
+                              "hd256-grp1-pos640-T300"])
+@pytest.mark.parametrize("ramp", [1.0, 40.0], ids=["flat", "rising-scores"])
+def test_flash_key_splits(shape, pos, T, ramp):
+    """A prompt step behind a seeded cache: few query units, so the flash
+    kernel splits the keys over workgroups and merges their partials; odd
+    positions put a split's first key past some of its tokens.  With rising
+    scores (keys up to 40 times larger towards the end) the reference of the
+    online softmax moves, so the output is rescaled mid-sweep."""
+    D, H, KV, hd, rot = shape
+    rng = np.random.default_rng(41)
+    w = _weights(rng, D, H, KV, hd)
+    K = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32) * np.geomspace(1.0, ramp, pos, dtype=np.float32)[None, :, None]
+    V = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32)
+    x = rng.normal(0, 1, (T, D)).astype(np.float32)
+    L = gdn.AttnLayer(new_li(), D, H, KV, hd, rot, 1e7, 1e-6, pos + T, w)
+    try:
+        L.cache_set(0, 0, pos, K, V)
+        got = L.forward(0, pos, x)
+    finally:
+        L.free()
+    ref = q.gated_attention(x, _ref_w(w), [K.transpose(1, 0, 2)], [V.transpose(1, 0, 2)], pos, H, KV, hd, rot, 1e7, 1e-6)
+    assert_close(got, ref, what=f"{shape} pos {pos} T {T} ramp {ramp}")
