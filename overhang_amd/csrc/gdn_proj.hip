@@ -2201,6 +2201,226 @@ void launch_i8(const ProjArgs &p, WvPlan w, const ProjArgs *f32, bool *f32_done,
     else launch_i8_tt<1, false>(p, w.G, nb, f, with, grid, nrg, ntt, per, st);
 }
 
+// ---------------------------------------------------------------- 5 to 16 tokens
+// A speculative step's draft tokens or a small batch: one launch, x read as
+// it is.  A workgroup is 8 waves on RT tiles of 16 rows, each wave an eighth
+// of k (NB blocks of 64) for all tokens (one 16-token MFMA operand); the
+// waves' sums meet in LDS in wave order.
+//   int8 rows, from the tiled copy (tile_q8), on the fp16 matrix cores
+//   (v_mfma_f32_16x16x32_f16, fp32 accumulation): the weights are exact in
+//   fp16, and each token's x over a chunk of at most 256 k, scaled by the
+//   power of two that takes its largest value below 2^12, is hi + lo with hi
+//   = fp16(x) and lo = fp16(x - hi): |x - hi - lo| <= 2^-22 |x| + 2^-37 of
+//   the chunk's largest (the split kernels' int8 planes: 2^-20 of the row's
+//   largest).  The chunk's sums go back by the exact power of two.  A wave
+//   requests its x first (L2), then all its weights (HBM), and splits x while
+//   the weights stream in.  Lane (l16, g) of 32-wide step s of a block holds
+//   row / token l16 at k = 16 g + 8 s + j.  H (up to 8 tokens): lanes l16 < 8
+//   hold and split one block of a token, lanes l16 >= 8 the next, so no lane
+//   repeats another's split; the second block's operand is the first's with
+//   the halves of its 16-lane rows exchanged (token columns past 7 are not read).
+//   fp32 rows (in_proj's b / a beside int8 rows, or a whole fp32 matrix):
+//   fp32 MFMA 16x16x4, lane (l16, g) at k = 16 i + 4 g + c for load i, so a
+//   load instruction reads 64 contiguous bytes of each of its 16 rows.
+// Bound by the weight stream and the launch, above 8 tokens by the split of x
+// that each workgroup does for itself.  35B shapes, T = 5: in_proj (25.7 MB)
+// 8.7 us and out_proj (8.4 MB) 5.9 us; T = 16: 12.3 and 11.5 us; the int8
+// planes' split launch and the split-queue kernel took 3.3 + 11.4 and 3.3 +
+// 13.2 us at either (out_proj 32 workgroups).  fp32 rows, T = 6: in_proj (101
+// MB) 27.1 and out_proj 14.1 us, against 30.7 and 15.6 us with k over 4 waves
+// and each row's loads in 16-byte pieces.
+constexpr int kFewTok = 16;
+constexpr int kFewWaves = 8;
+// k blocks of 64 per wave, or 0 where the kernel does not take the shape
+int few_blocks(int T, int I, int n_q) {
+    const int nb = I / (64 * kFewWaves);
+    if (T <= 4 || T > kFewTok || nb * 64 * kFewWaves != I || (nb != 1 && nb != 2 && nb != 4 && nb != 8)) return 0;
+    return n_q == 0 || tile_q8_wanted(n_q, I) ? nb : 0;
+}
+
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+// 8 int8 weights as fp16: the bytes of w + 128 under the high byte of 1024.0,
+// less 1152, every step exact
+__device__ __forceinline__ v8h q8_to_f16(unsigned lo, unsigned hi) {
+    const unsigned u[2] = {lo ^ 0x80808080u, hi ^ 0x80808080u};
+    const v2h off = {(_Float16)1152.f, (_Float16)1152.f};
+    v4u r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const unsigned m = __builtin_amdgcn_perm(0x64646464u, u[i / 2], i % 2 ? 0x04030402u : 0x04010400u);
+        r[i] = __builtin_bit_cast(unsigned, __builtin_bit_cast(v2h, m) - off);
+    }
+    return __builtin_bit_cast(v8h, r);
+}
+// 8 floats times sc as fp16 pairs: h = fp16(x sc), l = fp16(x sc - h)
+__device__ __forceinline__ void f16_split2(const v4f &a, const v4f &b, float sc, v4u &h, v4u &l) {
+    const float v[8] = {a[0] * sc, a[1] * sc, a[2] * sc, a[3] * sc, b[0] * sc, b[1] * sc, b[2] * sc, b[3] * sc};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const v2h x = {(_Float16)v[2 * j], (_Float16)v[2 * j + 1]};
+        const v2h r = {(_Float16)(v[2 * j] - (float)x[0]), (_Float16)(v[2 * j + 1] - (float)x[1])};
+        h[j] = __builtin_bit_cast(unsigned, x);
+        l[j] = __builtin_bit_cast(unsigned, r);
+    }
+}
+// v with the 8-lane halves of each 16-lane row exchanged
+__device__ __forceinline__ v4u ror8(const v4u &v) {
+    v4u r;
+#pragma unroll
+    for (int i = 0; i < 4; i++) r[i] = (unsigned)__builtin_amdgcn_update_dpp(0, (int)v[i], 0x128, 0xF, 0xF, false);
+    return r;
+}
+
+template <int NB, int RT, bool H>
+__global__ __launch_bounds__(kFewWaves * OMH_WAVE) void proj_few_kernel(const ProjArgs p, int nf) {
+    constexpr int CH = NB < 4 ? NB : 4;            // blocks whose x is held at once
+    constexpr int XB = H ? CH / 2 : CH;            // of those, blocks per lane
+    static_assert(!H || CH % 2 == 0, "blocks in pairs");
+    __shared__ v4f red[kFewWaves][RT][OMH_WAVE];
+    const int tid = threadIdx.x, lane = tid % OMH_WAVE, l16 = lane % 16, g = lane / 16;
+    const int wv = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
+    const int kbeg = wv * NB * 64;
+    const bool f32 = (int)blockIdx.x < nf;         // the fp32 rows' workgroups come first
+    const int t0 = f32 ? (int)blockIdx.x : ((int)blockIdx.x - nf) * RT;   // first row tile of its kind
+    const int nrow = f32 ? p.O - p.n_q : p.n_q, ntile = (nrow + 15) / 16;
+    v4f acc[RT];
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) acc[rt] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (f32) {
+        const float *xr = p.x + (size_t)min(l16, p.T - 1) * p.ldx + kbeg + 4 * g;
+        const float *wr = p.W + (size_t)min(16 * t0 + l16, nrow - 1) * p.I + kbeg + 4 * g;
+        v4f w[NB][4], odd = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int b = 0; b < NB; b++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) w[b][i] = *reinterpret_cast<const v4f *>(wr + 64 * b + 16 * i);
+#pragma unroll
+        for (int b = 0; b < NB; b++) {
+            v4f x[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = *reinterpret_cast<const v4f *>(xr + 64 * b + 16 * i);
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int c = 0; c < 4; c += 2) {
+                    acc[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][i][c], x[i][c], acc[0], 0, 0, 0);
+                    odd = __builtin_amdgcn_mfma_f32_16x16x4f32(w[b][i][c + 1], x[i][c + 1], odd, 0, 0, 0);
+                }
+        }
+        acc[0] += odd;
+    } else {
+        const float *xr = p.x + (size_t)min(H ? l16 % 8 : l16, p.T - 1) * p.ldx + kbeg + 16 * g + (H ? 64 * (l16 / 8) : 0);
+        v4i w[RT][NB];
+#pragma unroll
+        for (int c0 = 0; c0 < NB; c0 += CH) {
+            v4f x[XB][4];
+#pragma unroll
+            for (int b = 0; b < XB; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) x[b][i] = *reinterpret_cast<const v4f *>(xr + 64 * (c0 + (H ? 2 : 1) * b) + 4 * i);
+            __builtin_amdgcn_sched_barrier(0);     // x first, then the weights
+            if (c0 == 0) {
+#pragma unroll
+                for (int b = 0; b < NB; b++)
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++)
+                        w[rt][b] = *reinterpret_cast<const v4i *>(
+                            p.Qt + ((size_t)min(t0 + rt, ntile - 1) * (p.I / 64) + kbeg / 64 + b) * 1024 + 16 * lane);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+            // the token's largest |x| of the chunk; 2^(sf - 127) takes it into [2^11, 2^12)
+            float mx = 0.f;
+#pragma unroll
+            for (int b = 0; b < XB; b++)
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) mx = fmaxf(mx, fabsf(x[b][i][c]));
+            if constexpr (H) mx = fmaxf(mx, omh_dpp<0x128>(mx));
+            mx = omh_swap32_max(omh_swap16_max(mx));
+            const int sf = min(253, 265 - (int)(__builtin_bit_cast(unsigned, mx) >> 23));
+            const float sc = __builtin_bit_cast(float, sf << 23), back = __builtin_bit_cast(float, (254 - sf) << 23);
+            v4u h[XB][2], l[XB][2];
+#pragma unroll
+            for (int b = 0; b < XB; b++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) f16_split2(x[b][2 * s], x[b][2 * s + 1], sc, h[b][s], l[b][s]);
+            v4f sum[RT];
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++) sum[rt] = v4f{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int b = 0; b < CH; b++)
+#pragma unroll
+                for (int s = 0; s < 2; s++) {
+                    constexpr int P = H ? 2 : 1;
+                    const v4u hb = H && b % 2 ? ror8(h[b / P][s]) : h[b / P][s];
+                    const v4u lb = H && b % 2 ? ror8(l[b / P][s]) : l[b / P][s];
+#pragma unroll
+                    for (int rt = 0; rt < RT; rt++) {
+                        const v4i q = w[rt][c0 + b];
+                        const v8h a = q8_to_f16((unsigned)q[2 * s], (unsigned)q[2 * s + 1]);
+                        sum[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(v8h, lb), sum[rt], 0, 0, 0);
+                        sum[rt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(v8h, hb), sum[rt], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+            for (int rt = 0; rt < RT; rt++)
+#pragma unroll
+                for (int i = 0; i < 4; i++) acc[rt][i] = fmaf(sum[rt][i], back, acc[rt][i]);
+        }
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; rt++) red[wv][rt][lane] = acc[rt];
+    __syncthreads();
+    // lane (token l16, g) of tile rt: rows 4 g .. +3
+    const int rt = wv;
+    if (rt >= (f32 ? 1 : RT) || t0 + rt >= ntile || l16 >= p.T) return;
+    v4f r = red[0][rt][lane];
+#pragma unroll
+    for (int k = 1; k < kFewWaves; k++) r += red[k][rt][lane];
+    const int row = 16 * (t0 + rt) + 4 * g;
+    float *y = p.y + (size_t)l16 * p.ldy + (f32 ? p.n_q : 0) + row;
+    if (!f32) {
+        r *= *reinterpret_cast<const v4f *>(p.scale + row);
+        *reinterpret_cast<v4f *>(y) = r;
+    } else if (row + 3 < nrow) {
+        *reinterpret_cast<v4f *>(y) = r;
+    } else {
+        for (int i = 0; i < 4; i++)
+            if (row + i < nrow) y[i] = r[i];
+    }
+}
+
+template <int NB, int RT>
+void launch_few_rt(const ProjArgs &p, int nf, dim3 grid, hipStream_t st) {
+    const dim3 blk(kFewWaves * OMH_WAVE);
+    if constexpr (NB >= 2)
+        if (p.T <= 8) {
+            hipLaunchKernelGGL((proj_few_kernel<NB, RT, true>), grid, blk, 0, st, p, nf);
+            return;
+        }
+    hipLaunchKernelGGL((proj_few_kernel<NB, RT, false>), grid, blk, 0, st, p, nf);
+}
+template <int NB>
+void launch_few_nb(const ProjArgs &p, hipStream_t st) {
+    const int nf = (p.O - p.n_q + 15) / 16, tiles = (p.n_q + 15) / 16;
+    // row tiles per workgroup: as few as keep every workgroup resident at
+    // once, one per CU (a second round for a few of them would double the time)
+    const int rt = tiles == 0 ? 1 : std::min(4, (tiles + std::max(1, kCUs - nf) - 1) / std::max(1, kCUs - nf));
+    const dim3 grid(nf + (tiles + rt - 1) / rt);
+    if (rt == 1) launch_few_rt<NB, 1>(p, nf, grid, st);
+    else if (rt == 2) launch_few_rt<NB, 2>(p, nf, grid, st);
+    else if (rt == 3) launch_few_rt<NB, 3>(p, nf, grid, st);
+    else launch_few_rt<NB, 4>(p, nf, grid, st);
+}
+void launch_few(const ProjArgs &p, int nb, hipStream_t st) {
+    if (nb == 1) launch_few_nb<1>(p, st);
+    else if (nb == 2) launch_few_nb<2>(p, st);
+    else if (nb == 4) launch_few_nb<4>(p, st);
+    else launch_few_nb<8>(p, st);
+}
+
 inline bool al16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; }
 
 struct XbLayout {
@@ -2290,6 +2510,8 @@ size_t proj_xb_bytes(int T, int I, int n_q) { return xb_layout(T, I, n_q).total;
 
 bool proj_x_int8_planes(int T, int I, int n_q) { return use_i8(T, I, n_q); }
 
+bool proj_reads_x(int T, int I, int n_q) { return few_blocks(T, I, n_q) > 0; }
+
 hipError_t launch_proj(const ProjArgs &p, hipStream_t st) {
     if (p.O <= 0 || p.T <= 0) return hipSuccess;
     if (!proj_supported(p.I, p.n_q)) return hipErrorInvalidValue;
@@ -2316,6 +2538,12 @@ hipError_t launch_proj(const ProjArgs &p, hipStream_t st) {
         }
 #undef OMH_GEMV
 #undef OMH_GEMV_KS
+        return hipGetLastError();
+    }
+    // 5 to 16 tokens: one launch that reads x as it is
+    if (const int nb = few_blocks(p.T, p.I, p.n_q);
+        nb > 0 && !p.x_split && (p.n_q == 0 || p.Qt) && al16(p.x) && al16(p.y) && p.ldx % 4 == 0 && p.ldy % 4 == 0) {
+        launch_few(p, nb, st);
         return hipGetLastError();
     }
     // int8 rows on the bf16 matrix cores (bf16 x 3), the fp32 rows after

@@ -303,11 +303,15 @@ int decode_full_on(int li, int B, const float *x, float *out, hipStream_t st, ch
     HIP_OK(launch_proj(p, st));
     const int vh = L.d.vh;
     const float *zz = in + L.conv_dim, *bb = zz + L.vdim, *aa = bb + vh;
-    // the core writes out_proj's bf16 planes itself, saving the split launch;
+    // the core writes out_proj's planes itself, where it takes planes, saving the split launch;
     // at up to 4 tokens with int8 out_proj rows (the GEMV) the core runs as
     // column slices that leave the gated norm's 1 / rms to the GEMV instead
     const bool i8 = proj_x_int8_planes(B, L.vdim, L.out_nq);
-    uint16_t *planes = xb && L.out_nq > 0 && decode_planes_supported(L.d.vd, decode_variant(), i8) ? xb : nullptr;
+    // (up to 8 tokens an out_proj that splits x itself is the faster one:
+    // whole int8 step at the 35B shape 22.8 against 27.7 us at B = 5, but
+    // 34.1 us at 12 where B = 13 with the core's planes takes 31.4)
+    const bool reads_x = B <= 8 && proj_reads_x(B, L.vdim, L.out_nq);
+    uint16_t *planes = xb && L.out_nq > 0 && !reads_x && decode_planes_supported(L.d.vd, decode_variant(), i8) ? xb : nullptr;
     const int defer = B <= 4 && L.out_nq == D && !planes && decode_variant() == 0 && L.d.kh * B < 256
                           ? decode_deferred_slices(L.d.kd, L.d.vd) : 0;
     float *ssq = defer ? reinterpret_cast<float *>(scr + ds.ssq) : nullptr;

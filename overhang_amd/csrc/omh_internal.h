@@ -152,6 +152,8 @@ size_t proj_xb_bytes(int T, int I, int n_q);
 // whether that projection takes x as int8 planes (i8_off layout) rather than
 // bf16 planes (xpiece layout): what a kernel writing x ahead must produce
 bool proj_x_int8_planes(int T, int I, int n_q);
+// whether that projection reads x itself (5 to 16 tokens): no planes to write ahead
+bool proj_reads_x(int T, int I, int n_q);
 // hidden size I and int8 row count n_q the projection kernels take
 bool proj_supported(int I, int n_q);
 hipError_t launch_proj(const ProjArgs &p, hipStream_t st);

@@ -12,7 +12,7 @@ import pytest
 
 import oracle
 from overhang_amd import gdn, synth
-from overhang_amd.dims import CFG1, TINY, Q35B
+from overhang_amd.dims import CFG1, TINY, Q35B, GdnDims
 from tests.tol import assert_close
 
 pytestmark = pytest.mark.gpu
@@ -299,3 +299,35 @@ def test_int8_decode_batch_kernel_matches_stream_kernel(shape, B, monkeypatch):
         L.free()
     assert_close(outs["1"][0], outs["0"][0], atol=2e-5, rtol=2e-5, what=f"B={B} split-queue vs stream out")
     assert_close(outs["1"][1], outs["0"][1], atol=2e-5, rtol=2e-5, what=f"B={B} split-queue vs stream S")
+
+
+@pytest.mark.parametrize("shape", [(16, 32, 128, 128, 2048), (4, 8, 64, 64, 1024), (3, 6, 64, 64, 512)],
+                         ids=["35b", "k1024-k512", "k512-6heads"])
+@pytest.mark.parametrize("int8", [True, False], ids=["int8", "f32"])
+@pytest.mark.parametrize("B", [5, 8, 9, 12, 13, 16])
+def test_few_token_projections(shape, int8, B):
+    """5 to 16 tokens: the projections that split x themselves (up to 8 tokens
+    two k blocks per 16 lanes, above that one), with k over 8 waves in 1 to 8
+    blocks each, rows that end inside a workgroup's tiles and fp32 rows that
+    end inside a tile; tokens from 1e-3 to 10 in size, since each is scaled
+    by its own largest value.  (The output grows with the gate silu(z), so with
+    x: at 1e3 its rms is about 600 and fp32 sums in another order, 1e-5 of
+    that, pass the absolute 2e-3; at 10 they stay below 1e-4.)"""
+    kh, vh, kd, vd, hidden = shape
+    d = GdnDims(kh=kh, vh=vh, kd=kd, vd=vd, K=4, hidden=hidden)
+    w = synth.layer_weights(d, 3)
+    x = synth.normal(5, synth.S_X, (B, hidden)) * np.geomspace(1e-3, 10, B, dtype=np.float32)[:, None]
+    x[1, 7] = 0.0
+    if B > 9:
+        x[9] = 0.0
+    conv0, S0 = synth.states(d, 4, B=B)
+    L = gdn.GdnLayer(new_li(), d, w, max_seqs=B, int8=int8)
+    try:
+        for b in range(B):
+            L.set_state(b, conv0[b], S0[b])
+        out = L.decode(x)
+    finally:
+        L.free()
+    for b in range(B) if kh < 16 else (0, 1, B - 1):
+        ref, _, _ = oracle.layer_seq(d, w, x[b:b + 1], conv0[b], S0[b], int8=int8)
+        assert_close(out[b:b + 1], ref, what=f"{shape} int8={int8} token {b} of {B}")
