@@ -11,7 +11,9 @@
 //     S <- e^{gc_last} S + (K * e^{gc_last - gc})^T v_new
 // Only exp of differences of cumulative decays are formed, never exp(-gc).
 //
-// Three launches, all on the caller's stream:
+// Steps of up to kFewTokens tokens run the recurrence token by token in one
+// launch (prefill_few_kernel).  Longer ones are three launches, all on the
+// caller's stream:
 //   P1 wy      per (key head, chunk) with its value heads: conv + SiLU, q/k
 //              L2 norm, gates, KK^T, QK^T, (I+L)^-1 blocks, W, U on fp32
 //              MFMA, written as per-lane fragment panels           MFMA-bound
@@ -995,6 +997,190 @@ void prefill_scan_kernel(const PrefillArgs a) {
         for (int r = 0; r < 4; r++) Sbase[(size_t)(16 * w + 4 * g4 + r) * D + 16 * cb + l16] = S[r];
 }
 
+// ---------------------------------------------------------------- few tokens
+// Up to kFewTokens tokens (a speculative step's draft, a short turn): the
+// recurrence itself, one token after another, in one launch.  A 64-token
+// chunk costs its WY item, its scan step and two more launches however few of
+// its tokens are live (35B, any T <= 64: 28.9 + 7.4 + 4.1 us); one token of
+// the recurrence costs 0.5 us here, on top of 6 us for the launch, the state's
+// loads and the conv.  What bounds it is that chain: each SIMD runs two waves'
+// products of one token (128 a lane), then the lane sums.
+//
+// One workgroup per value head.  Wave w holds the state's columns 16 w .. +15
+// in registers, lane (l16, g) column l16 at rows 16 i + 4 g + c, so a column's
+// sums are within a wave (two lane swaps) and a token needs no barrier; its k
+// and q come from LDS, four 16-byte broadcasts a time without a bank
+// conflict.  Conv, gates and norm factors of all tokens are formed up front,
+// the gated norm at the end.  As in the decode kernels both sums use the old
+// state: kv = gamma S^T k, delta = beta (v - kv), o = gamma S^T q + (k.q) delta.
+//
+// The conv history: a q / k channel's is read by all rep value heads of the
+// key head, so the last of them to have read it (an arrival counter that it
+// resets) commits the new inputs; v channels are the workgroup's own.
+constexpr int kFewTokens = 40;
+template <int D>
+struct FewShape {
+    static constexpr int NW = D / 16, NT = NW * OMH_WAVE;   // one wave per 16 columns
+    static constexpr int NI = D / 16;                       // 16-row groups (4 rows per lane)
+    static constexpr int ZN = (kFewTokens * D + NT - 1) / NT;   // outputs per thread
+    static_assert(NT >= 3 * D && NT % D == 0 && NT >= kFewTokens, "a conv channel per thread, an output column per thread");
+    // q, k, v (then o) per token; gamma, beta, rk, rq, kq; the waves' sums of o^2
+    static __host__ __device__ constexpr size_t lds(int T) { return (size_t)T * (3 * D + 8 + NW) * sizeof(float); }
+};
+
+template <int D>
+__global__ __launch_bounds__(FewShape<D>::NT) void prefill_few_kernel(const PrefillArgs a, int conv_dim) {
+    using F = FewShape<D>;
+    constexpr int NW = F::NW, NT = F::NT, NI = F::NI, ZN = F::ZN;
+    extern __shared__ __attribute__((aligned(16))) float few[];
+    const int T = a.T, rep = a.vh / a.kh, h = blockIdx.x, hk = h / rep, K = a.K;
+    float *qs = few, *ks = qs + T * D, *vs = ks + T * D, *fac = vs + T * D, *ssq = fac + 8 * T;
+    __shared__ int s_last;
+    const int tid = threadIdx.x, lane = tid % OMH_WAVE, l16 = lane % 16, g = lane / 16;
+    const int w = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
+    const LayerPtrs &L = a.L;
+    const int ph = L.phase[L.epoch * L.max_seqs + a.seq];
+
+    // the state (rows 16 i + 4 g + c of column 16 w + l16)
+    float *Sp = L.S + ((size_t)a.seq * a.vh + h) * D * D + (size_t)(4 * g) * D + 16 * w + l16;
+    float s[NI][4];
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) s[i][c] = Sp[(size_t)(16 * i + c) * D];
+
+    // conv + SiLU (qwen.c:311-319) of channel tid: q and k of the key head, v of this head
+    const bool conv = tid < 3 * D;
+    const int part = tid / D, ci = tid % D;
+    const int gch = part == 0 ? hk * D + ci : (part == 1 ? (a.kh + hk) * D + ci : 2 * a.kh * D + h * D + ci);
+    float hist[3] = {0.f, 0.f, 0.f};                // the last three inputs, oldest first
+    if (conv) {
+        const float4 wt = *reinterpret_cast<const float4 *>(L.conv_w + (size_t)gch * kConvRing);
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+            hist[m] = m >= kConvRing - K ? L.conv_st[ring_at(a.seq, (ph + 1 + m) & (kConvRing - 1), gch, conv_dim)] : 0.f;
+        float *dst = (part == 0 ? qs : (part == 1 ? ks : vs)) + ci;
+        constexpr int XB = 8;
+        for (int t0 = 0; t0 < T; t0 += XB) {
+            float x[XB];
+#pragma unroll
+            for (int j = 0; j < XB; j++) x[j] = a.qkv[(size_t)min(t0 + j, T - 1) * a.ld_qkv + gch];
+#pragma unroll
+            for (int j = 0; j < XB; j++)
+                if (t0 + j < T) {
+                    float acc = 0.f;
+                    if (K >= 4) acc += wt.x * hist[0];
+                    if (K >= 3) acc += wt.y * hist[1];
+                    acc += wt.z * hist[2];
+                    acc += wt.w * x[j];
+                    hist[0] = hist[1];
+                    hist[1] = hist[2];
+                    hist[2] = x[j];
+                    dst[(t0 + j) * D] = omh_silu_fast(acc);
+                }
+        }
+    }
+    if (tid < T) {                                  // the gates (qwen.c:324-325, 334-337)
+        const float gl = -expf(L.A_log[h]) * omh_softplus(a.a[(size_t)tid * a.ld_ab + h] + L.dt_bias[h]);
+        fac[8 * tid] = expf(gl);
+        fac[8 * tid + 1] = omh_sigmoid(a.b[(size_t)tid * a.ld_ab + h]);
+    }
+    // the output gate's inputs and the norm weight, requested ahead
+    float zr[ZN];
+#pragma unroll
+    for (int j = 0; j < ZN; j++) zr[j] = a.z[(size_t)min((tid + NT * j) / D, T - 1) * a.ld_z + (size_t)h * D + tid % D];
+    const float gn = L.gnorm[tid % D];
+    __syncthreads();
+
+    // norm factors (qwen.c:153-157, 326-329), a wave per token
+    for (int t = w; t < T; t += NW) {
+        float sq = 0.f, sk = 0.f, qk = 0.f;
+        for (int i = lane; i < D; i += OMH_WAVE) {
+            const float q = qs[t * D + i], k = ks[t * D + i];
+            sq += q * q;
+            sk += k * k;
+            qk += q * k;
+        }
+        sq = omh_lane_sum_below<OMH_WAVE>(sq);
+        sk = omh_lane_sum_below<OMH_WAVE>(sk);
+        qk = omh_lane_sum_below<OMH_WAVE>(qk);
+        if (lane == 0) {
+            const float rq = 1.f / sqrtf(sq + 1e-6f) * (1.f / sqrtf((float)D)), rk = 1.f / sqrtf(sk + 1e-6f);
+            fac[8 * t + 2] = rk;
+            fac[8 * t + 3] = rq;
+            fac[8 * t + 4] = qk * rq * rk;
+        }
+    }
+    if (tid == 0) {
+        // (every thread's history reads are behind the barrier above)
+        int *cnt = L.cnt + (size_t)a.seq * a.vh + hk;
+        s_last = __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == rep - 1;
+        if (s_last) __hip_atomic_store(cnt, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (conv && (part == 2 || s_last))
+#pragma unroll
+        for (int m = 0; m < 3; m++)
+            if (m >= kConvRing - K && T - 3 + m >= 0)
+                L.conv_st[ring_at(a.seq, (ph + T - 3 + m) & (kConvRing - 1), gch, conv_dim)] = hist[m];
+    if (h == 0)
+        for (int b = tid; b < L.max_seqs; b += NT)
+            L.phase[(1 - L.epoch) * L.max_seqs + b] =
+                b == a.seq ? (ph + T) & (kConvRing - 1) : L.phase[L.epoch * L.max_seqs + b];
+
+    for (int t = 0; t < T; t++) {
+        const float4 f0 = *reinterpret_cast<const float4 *>(fac + 8 * t);
+        const float gam = f0.x, beta = f0.y, rk = f0.z, rq = f0.w, kq = fac[8 * t + 4];
+        const float v = vs[t * D + 16 * w + l16];
+        const float *kp = ks + t * D + 4 * g, *qp = qs + t * D + 4 * g;
+        float4 k[NI];
+        float ak = 0.f, aq = 0.f, bk = 0.f, bq = 0.f;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            k[i] = *reinterpret_cast<const float4 *>(kp + 16 * i);
+            const float4 q = *reinterpret_cast<const float4 *>(qp + 16 * i);
+            ak = fmaf(s[i][0], k[i].x, ak);
+            bk = fmaf(s[i][1], k[i].y, bk);
+            aq = fmaf(s[i][0], q.x, aq);
+            bq = fmaf(s[i][1], q.y, bq);
+            ak = fmaf(s[i][2], k[i].z, ak);
+            bk = fmaf(s[i][3], k[i].w, bk);
+            aq = fmaf(s[i][2], q.z, aq);
+            bq = fmaf(s[i][3], q.w, bq);
+        }
+        const float sk = omh_swap32_sum(omh_swap16_sum(ak + bk)), sq = omh_swap32_sum(omh_swap16_sum(aq + bq));
+        const float delta = beta * (v - gam * rk * sk);
+        const float o = fmaf(delta, kq, gam * rq * sq), d2 = rk * delta;
+#pragma unroll
+        for (int i = 0; i < NI; i++) {
+            s[i][0] = fmaf(d2, k[i].x, gam * s[i][0]);
+            s[i][1] = fmaf(d2, k[i].y, gam * s[i][1]);
+            s[i][2] = fmaf(d2, k[i].z, gam * s[i][2]);
+            s[i][3] = fmaf(d2, k[i].w, gam * s[i][3]);
+        }
+        const float oo = omh_lane_sum_below<16>(o * o);
+        if (g == 0) vs[t * D + 16 * w + l16] = o;   // (this column's v has been read by its wave)
+        if (lane == 0) ssq[t * NW + w] = oo;
+    }
+#pragma unroll
+    for (int i = 0; i < NI; i++)
+#pragma unroll
+        for (int c = 0; c < 4; c++) Sp[(size_t)(16 * i + c) * D] = s[i][c];
+    __syncthreads();
+
+    // the gated norm (qwen.c:353-357)
+#pragma unroll
+    for (int j = 0; j < ZN; j++) {
+        const int t = (tid + NT * j) / D;
+        if (t >= T) break;
+        float ss = 0.f;
+#pragma unroll
+        for (int i = 0; i < NW; i++) ss += ssq[t * NW + i];
+        const float rn = 1.f / sqrtf(ss / (float)D + a.eps);
+        a.core[((size_t)t * a.vh + h) * D + tid % D] = vs[t * D + tid % D] * rn * gn * omh_silu(zr[j]);
+    }
+}
+
 size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 
 // Workgroups of the persistent WY kernel: the device's CU count.
@@ -1011,6 +1197,10 @@ int wy_grid() {
 template <int D>
 hipError_t launch_prefill_d(const PrefillArgs &a, hipStream_t st) {
     const int conv_dim = 2 * a.kh * D + a.vh * D;
+    if (!prefill_chunked(a.T)) {
+        hipLaunchKernelGGL((prefill_few_kernel<D>), dim3(a.vh), dim3(FewShape<D>::NT), FewShape<D>::lds(a.T), st, a, conv_dim);
+        return hipGetLastError();
+    }
     // persistent: one workgroup per CU (the LDS footprint allows one), a
     // multiple of 8 so the XCD-aware item order holds
     const int rep = a.vh / a.kh;
@@ -1040,6 +1230,8 @@ bool set_lds_limit() {
 }
 
 }  // namespace
+
+bool prefill_chunked(int T) { return T > kFewTokens; }
 
 size_t prefill_scratch_bytes(int D, int kh, int vh, int T) {
     const size_t Tp = (size_t)((T + C - 1) / C) * C, nc = Tp / C;

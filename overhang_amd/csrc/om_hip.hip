@@ -382,8 +382,10 @@ int prefill_core(int li, int seq, int T, const float *qkv, int64_t ld_qkv, const
     A.L = ptrs(L);
     A.seq = seq; A.T = T; A.nc = (T + kChunk - 1) / kChunk; A.Tp = A.nc * kChunk;
     A.kh = d.kh; A.vh = d.vh; A.K = d.conv_k; A.eps = d.eps;
-    if (int rc = ensure(g_pre, prefill_scratch_bytes(D, d.kh, d.vh, T))) return rc;
-    prefill_bind_scratch(A, D, g_pre.p);
+    if (prefill_chunked(T)) {
+        if (int rc = ensure(g_pre, prefill_scratch_bytes(D, d.kh, d.vh, T))) return rc;
+        prefill_bind_scratch(A, D, g_pre.p);
+    }
     HIP_OK(launch_prefill_core(A, D, st));
     L.epoch ^= 1;                      // the conv commit wrote the other phase buffer
     return OMH_OK;

@@ -186,6 +186,8 @@ struct PrefillArgs {
     float *pw, *pa, *pu;                 // per (value head, chunk) operand panels (WY kernel -> scan)
     float *pq, *pk;                      // q^, k^ per (key head, chunk), shared by its value heads
 };
+// whether a step of T tokens runs chunk-wise (and takes the scratch)
+bool prefill_chunked(int T);
 size_t prefill_scratch_bytes(int D, int kh, int vh, int T);
 void prefill_bind_scratch(PrefillArgs &a, int D, void *base);
 bool prefill_supported(int kd, int vd, int rep, int K);

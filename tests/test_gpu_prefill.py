@@ -297,3 +297,38 @@ def test_long_warm_append_35b_split_invariance(split):
         assert_close(Sb, Sa, what=f"split {split} S")
     A.free()
     B.free()
+
+
+@pytest.mark.parametrize("kh,vh,D,K", [(2, 4, 16, 4), (1, 3, 32, 4), (2, 2, 64, 3), (2, 8, 128, 4), (1, 2, 128, 2)])
+@pytest.mark.parametrize("T", [2, 7, 8, 9, 17, 40, 41])
+def test_few_token_prefill(kh, vh, D, K, T):
+    """Up to 40 tokens run the recurrence token by token in one launch, 41 and
+    more chunk-wise: two such steps in a row and a decode step, on the second
+    of three sequences, so that the conv history each leaves (committed by the
+    last value head of a key head to have read it) and its ring phase are
+    taken up by the next and the other sequences are left as they were."""
+    d = GdnDims(kh, vh, D, D, K, 0)
+    seed = 5000 + 7 * kh + vh + D + K + T
+    w = synth.layer_weights(d, seed, gnorm_std=0.1, projections=False)
+    conv0, S0 = synth.states(d, seed)
+    L = gdn.GdnLayer(new_li(), d, w, max_seqs=3)
+    for s in range(3):
+        L.set_state(s, conv0, S0)
+    inp = synth.core_inputs(d, 2 * T, seed)
+    got = [L.prefill_core(1, *(inp[k][i:i + T] for k in ("qkv", "z", "a", "b"))) for i in (0, T)]
+    ref, cref, Sref = oracle.core_seq(d, w, inp["qkv"], inp["z"], inp["a"], inp["b"], conv0, S0)
+    what = f"kh={kh} vh={vh} D={D} K={K} T={T}"
+    assert_close(np.concatenate(got), ref, what=what + " core")
+    for s in range(3):
+        conv, S = L.get_state(s)
+        if s == 1:
+            assert_close(S, Sref, what=what + " S")
+            assert np.array_equal(conv, cref), "conv history is a copy of the inputs"
+        else:
+            assert np.array_equal(conv, conv0) and np.array_equal(S, S0), f"sequence {s} changed"
+    one = synth.core_inputs(d, 3, seed + 1)
+    out = L.decode_core(one["qkv"], one["z"], one["a"], one["b"])
+    for s, (c, S) in enumerate([(conv0, S0), (cref, Sref), (conv0, S0)]):
+        r, _, _ = oracle.core_seq(d, w, *(one[k][s:s + 1] for k in ("qkv", "z", "a", "b")), c, S)
+        assert_close(out[s:s + 1], r, what=what + f" decode of sequence {s}")
+    L.free()
