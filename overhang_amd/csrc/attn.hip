@@ -12,13 +12,13 @@
 //     rot dims as two non-interleaved halves (qwen.c:388-398, inverse
 //     frequencies computed on the host as there), then q into a scratch row
 //     and k, v into the sequence's cache rows pos + t (qwen.c:400-404).
-//  2. the split kernel, flash-decoding: one workgroup per (key split, kv
-//     head, token) reads the split's K and V rows once for all the query
-//     heads of its group (GQA, qwen.c:408-409), keeps a running max and sum
-//     per head (online softmax) and writes unnormalised partials.  Head
-//     widths of 64 and more: attn_split_mfma_kernel, K and V from HBM
-//     straight into fp32 MFMA operands (the heads of the group are the
-//     products' 16 columns).  Width 32: attn_split_kernel, 64-key tiles
+//  2. the split kernel, flash-decoding: a workgroup reads the K and V rows of
+//     one key split of one kv head once for the query heads of its group
+//     (GQA, qwen.c:408-409), keeps a running max and sum per head (online
+//     softmax) and writes unnormalised partials.  Head widths of 64 and
+//     more: attn_split_mfma_kernel, K and V from HBM straight into fp32 MFMA
+//     operands whose 16 columns are (token, head) pairs of the group.  Width
+//     32: attn_split_kernel, a workgroup per token, 64-key tiles
 //     staged through LDS, lane = key for the scores (q broadcast from LDS),
 //     lane = 4 output columns for P.V (each key's weight by readlane).
 //  3. attn_combine_kernel, per (token, head, 64 columns): merges the splits,
@@ -26,8 +26,8 @@
 // The o_proj is a second launch_proj.
 //
 // Decode is HBM-bound on the visible cache: 2 * KV * n * hd * 4 bytes for
-// n = pos + 1 keys; the splits give >= 256 workgroups (one per CU, as the
-// LDS footprint allows).  Token t
+// n = pos + 1 keys; the splits fill the CUs once (one workgroup per CU, as
+// the LDS footprint allows).  Token t
 // sees keys 0 .. pos+t (causal), and the key tiles beyond that are masked.
 #include "omh_internal.h"
 #include "omh_device.h"
@@ -124,7 +124,8 @@ __device__ __forceinline__ void prep_row(const AttnArgs &a, const float *src, co
     prep_row_regs<HD>(a, v, wv, w != nullptr, row, lane, cs_t, sn_t);
 }
 
-// The prep: one workgroup of kPrepWaves waves per token.  The token's RoPE
+// The prep: one workgroup of kPrepWaves waves per token (gridDim.y of them
+// where tokens are few, each with its share of the rows).  The token's RoPE
 // cos and sin (rot / 2 frequencies) go into LDS once, then wave w takes rows
 // w, w + kPrepWaves, ... of [H q heads, KV k heads, KV v heads]: q into the
 // scratch, k and v into the cache rows pos + t.  A wave's next row (and its
@@ -138,6 +139,7 @@ __global__ __launch_bounds__(kPrepWaves * OMH_WAVE) void attn_prep_kernel(const 
     const int H = a.H, KV = a.KV, nr = H + 2 * KV;
     const int t = blockIdx.x, tid = threadIdx.x, lane = tid % OMH_WAVE;
     const int wv = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
+    const int r0 = wv + kPrepWaves * blockIdx.y, rs = kPrepWaves * gridDim.y;   // this wave's first row, and the step
     const int p = a.pos + t;
     const float *row = a.qkv + (size_t)t * a.ld_qkv;
     // row r's source and norm weights (null: a v row, copied)
@@ -158,17 +160,17 @@ __global__ __launch_bounds__(kPrepWaves * OMH_WAVE) void attn_prep_kernel(const 
             wt[i] = w && j < HD ? w[j] : 0.f;
         }
     };
-    if (wv < nr) fetch(wv);
+    if (r0 < nr) fetch(r0);
     rope_table(a, p, cs, sn, tid, kPrepWaves * OMH_WAVE);
     __syncthreads();
-    for (int r = wv; r < nr; r += kPrepWaves) {
+    for (int r = r0; r < nr; r += rs) {
         float cv[NE], cw[NE];
 #pragma unroll
         for (int i = 0; i < NE; i++) {
             cv[i] = v[i];
             cw[i] = wt[i];
         }
-        if (r + kPrepWaves < nr) fetch(r + kPrepWaves);
+        if (r + rs < nr) fetch(r + rs);
         float *dst;
         if (r < H) dst = a.qb + ((size_t)t * H + r) * HD;
         else if (r < H + KV) dst = a.Kc + (((size_t)a.seq * KV + (r - H)) * a.max_t + p) * HD;
@@ -377,18 +379,24 @@ void attn_split_kernel(const AttnArgs a) {   // one workgroup per CU (LDS): all 
 #undef OMH_ATTN_LOAD_PIECE
 
 // ---------------------------------------------------------------- decode on the matrix cores
-// The split kernel for head widths of 64 and more: the same work unit (one
-// key split of one kv head for one token, the prep folded in for decode
-// steps), with K and V going from HBM straight into fp32 MFMA operands, so
-// every key row is read once for all the group's query heads (no LDS
-// staging, no per-head re-reads).  Each of the NW waves streams its own
-// 16-key blocks (blocks w, w + NW, ...) and keeps its own online softmax.
+// The split kernel for head widths of 64 and more: one workgroup takes one
+// key split of one kv head for a column tile of 16 (token, query head) pairs
+// of its group (a decode step: the one token's heads, the prep folded in),
+// with K and V going from HBM straight into fp32 MFMA operands, so every key
+// row is read once for the 16 columns (no LDS staging, no per-head re-reads).
+// Steps of 2 to 63 tokens took a workgroup per token before, 8 of the 16
+// columns in use at 8 heads a group and the cache read again for every token:
+// 5 tokens at position 8001 (16 heads on 2 kv heads, width 256) 47.3 us (260
+// workgroups, two rounds of the CUs), as column tiles 21.3 us (252).  Tried:
+// a block's K and V rows in registers of their own, the next block's loads
+// ahead: 25.5 us (and a decode step at position 32767 37.0 us for 34.4).
+// Each of the NW waves streams its own 16-key blocks (blocks w, w + NW, ...) and keeps its own online softmax.
 // A wave holds one operand set: a block's K rows, then (once the scores are
 // formed) its V rows in the same registers; the two waves of a SIMD overlap
 // one's loads with the other's products:
 //   S^T = K Q^T   (v_mfma_f32_16x16x4_f32; A = K rows, lane l16 = key;
-//                  B = q from LDS, lane l16 = query head of the group, heads
-//                  past the group zero; head dims taken in the order 16 i + 4 g + s
+//                  B = q from LDS, lane l16 = column, columns past
+//                  the tile's last zero; head dims taken in the order 16 i + 4 g + s
 //                  on both operands, one 16-byte K load per 4 products),
 //   O += P V      (A = the probabilities as the score product left them:
 //                  key 4 g + s of lane group g is register s; B = V rows
@@ -396,8 +404,9 @@ void attn_split_kernel(const AttnArgs a) {   // one workgroup per CU (LDS): all 
 //                  tile 4 q + c, so one 16-byte V load serves 4 tiles).
 // The waves' (max, sum, O) then merge through LDS into the split's partial,
 // which the combine kernel merges with the other splits as before.  Keys
-// past the split's end or the token's position are masked (their rows
-// repeat a visible row, so every operand is finite).
+// past the split's end (their rows repeat its last one) and keys past a
+// column's own position are masked; values that are not finite reach only
+// the tokens that see them.
 template <int HD>
 struct MfmaSplitShape {
     static constexpr int NW = 8;                   // waves, two per SIMD
@@ -408,8 +417,10 @@ struct MfmaSplitShape {
     static_assert(HD % 64 == 0, "64-column V groups");
 };
 
-__device__ __forceinline__ omh_v4f ld_stream_v4(__amdgpu_buffer_rsrc_t r, int off) {
-    return __builtin_bit_cast(omh_v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, kOmhNT));
+// NT: streamed past the caches (one reader)
+template <bool NT>
+__device__ __forceinline__ omh_v4f ld_buf_v4(__amdgpu_buffer_rsrc_t r, int off) {
+    return __builtin_bit_cast(omh_v4f, __builtin_amdgcn_raw_buffer_load_b128(r, off, 0, NT ? kOmhNT : 0));
 }
 
 template <int HD, bool PREP>
@@ -418,21 +429,38 @@ void attn_split_mfma_kernel(const AttnArgs a) {
     using S = MfmaSplitShape<HD>;
     constexpr int NW = S::NW, NT = NW * OMH_WAVE, QS = S::QS, NI = S::NI, NQ = S::NQ;
     extern __shared__ float smem[];
-    float *qs = smem;                              // [kAttnMaxGroup][QS] the group's q rows
+    float *qs = smem;                              // [kAttnMaxGroup][QS] the columns' q rows
     float *mo = qs + kAttnMaxGroup * QS;           // [NW][16][HD] the waves' outputs (the prep's scratch before)
     float *mm = mo + NW * 16 * HD;                 // [NW][16] running max, then [NW][16] sums
 
     const int H = a.H, KV = a.KV, grp = H / KV, ns = a.ns;
-    const int s = blockIdx.x % ns, g = (blockIdx.x / ns) % KV, t = blockIdx.x / (ns * KV);
+    // unit (key split s, kv head g) and column tile ct; a unit's tiles run
+    // side by side on one XCD (workgroup i on XCD i mod 8), which then reads
+    // the unit's keys from memory once
+    const int nct = (a.T * grp + 15) / 16, nu = ns * KV;
+    const int ct = nu % 8 == 0 ? (int)blockIdx.x / 8 % nct : (int)blockIdx.x % nct;
+    const int unit = nu % 8 == 0 ? (int)blockIdx.x / (8 * nct) * 8 + (int)blockIdx.x % 8 : (int)blockIdx.x / nct;
+    const int s = unit % ns, g = unit / ns;
     const int tid = threadIdx.x, lane = tid % OMH_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
     const int l16 = lane % 16, g4 = lane / 16;
-    const int n = a.pos + t + 1;                   // keys token t sees
+    // column c of the tile is (token, head) pair c0 + c of the group's
+    // T * grp, head fastest (the quotient by a reciprocal: fewer than 2^10
+    // pairs and 16 heads, so the half keeps every one clear of rounding)
+    const float rgrp = __builtin_amdgcn_rcpf((float)grp);
+    auto token_of = [&](int c) __attribute__((always_inline)) { return (int)(((float)c + 0.5f) * rgrp); };
+    const int c0 = 16 * ct, ncol = min(16, a.T * grp - c0);
+    const int tlast = token_of(c0 + ncol - 1);
+    const int n = a.pos + tlast + 1;               // keys the tile's last token sees
     const int k0 = s * a.kps, k1 = min(n, k0 + a.kps);
-    const size_t pb = ((size_t)t * H + (size_t)g * grp) * ns + s;
+    // partial and q row of column c
+    auto row_of = [&](int c) __attribute__((always_inline)) {
+        const int t = token_of(c0 + c);
+        return (size_t)(t * H + g * grp + c0 + c - t * grp);
+    };
     if (k0 >= k1) {                                // an empty split: weight zero in the merge
-        for (int e = tid; e < grp * (HD / 4); e += NT) {
-            const size_t pi = pb + (size_t)(e / (HD / 4)) * ns;
+        for (int e = tid; e < ncol * (HD / 4); e += NT) {
+            const size_t pi = row_of(e / (HD / 4)) * ns + s;
             *reinterpret_cast<float4 *>(a.po + pi * HD + 4 * (e % (HD / 4))) = f4_zero();
             if (e % (HD / 4) == 0) {
                 a.pml[2 * pi] = -INFINITY;
@@ -453,14 +481,14 @@ void attn_split_mfma_kernel(const AttnArgs a) {
     auto load_k = [&](int b) __attribute__((always_inline)) {
         const int kk = min(k0 + 16 * b + l16, k1 - 1);
 #pragma unroll
-        for (int i = 0; i < NI; i++) kv[i] = ld_stream_v4(krs, (kk * HD + 16 * i + 4 * g4) * 4);
+        for (int i = 0; i < NI; i++) kv[i] = ld_buf_v4<PREP>(krs, (kk * HD + 16 * i + 4 * g4) * 4);
     };
     auto load_v = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             const int kr = min(k0 + 16 * b + 4 * g4 + st, k1 - 1);
 #pragma unroll
-            for (int q = 0; q < NQ; q++) kv[NQ * st + q] = ld_stream_v4(vrs, (kr * HD + 64 * q + 4 * l16) * 4);
+            for (int q = 0; q < NQ; q++) kv[NQ * st + q] = ld_buf_v4<PREP>(vrs, (kr * HD + 64 * q + 4 * l16) * 4);
         }
     };
     // Prologue.  A decode step's RoPE table comes first (its out-of-line
@@ -471,9 +499,10 @@ void attn_split_mfma_kernel(const AttnArgs a) {
     // straight-line code: loads complete in issue order, so the prep's waits
     // leave the block's loads in flight.  A prompt step's prepared q rows go
     // to LDS before the block loads.
-    const int p = a.pos + t;
+    // (decode steps: one token, its group's heads in one tile)
+    const int p = a.pos;
     if constexpr (PREP) {
-        const float *row = a.qkv + (size_t)t * a.ld_qkv;
+        const float *row = a.qkv;
         float *krow = mo, *cs = mo + HD, *sn = cs + HD / 2;
         rope_table(a, p, cs, sn, tid, NT);
         __syncthreads();
@@ -509,32 +538,33 @@ void attn_split_mfma_kernel(const AttnArgs a) {
         }
         load_k(wave);
     } else {
-        for (int e = tid; e < grp * (HD / 4); e += NT) {
+        for (int e = tid; e < ncol * (HD / 4); e += NT) {
             const int i = e / (HD / 4), c = e % (HD / 4);
             *reinterpret_cast<float4 *>(qs + i * QS + 4 * c) =
-                *reinterpret_cast<const float4 *>(a.qb + ((size_t)t * H + (size_t)g * grp + i) * HD + 4 * c);
+                *reinterpret_cast<const float4 *>(a.qb + row_of(i) * HD + 4 * c);
         }
         load_k(wave);
     }
     // (LDS-only barriers from here on: a full __syncthreads would also wait
     // for the block loads in flight)
     omh_lds_barrier();
-    // q as the B operand: lane (g4, head l16) reads q[l16][16 i + 4 g4 .. +3]
-    // (rows past the group read as zero)
-    if (grp < 16) {
-        for (int e = tid; e < (16 - grp) * (HD / 4); e += NT)
-            *reinterpret_cast<float4 *>(qs + (grp + e / (HD / 4)) * QS + 4 * (e % (HD / 4))) = f4_zero();
+    // q as the B operand: lane (g4, column l16) reads q[l16][16 i + 4 g4 .. +3]
+    // (columns past the tile's last read as zero)
+    if (ncol < 16) {
+        for (int e = tid; e < (16 - ncol) * (HD / 4); e += NT)
+            *reinterpret_cast<float4 *>(qs + (ncol + e / (HD / 4)) * QS + 4 * (e % (HD / 4))) = f4_zero();
         omh_lds_barrier();
     }
+    const int kend = min(k1, a.pos + token_of(c0 + min(l16, ncol - 1)) + 1);   // keys this lane's column sees end here
     const float *qrow = qs + l16 * QS + 4 * g4;
 
-    float m = -INFINITY, l = 0.f;                  // of head l16 (the same in the four lane groups)
+    float m = -INFINITY, l = 0.f;                  // of column l16 (the same in the four lane groups)
     omh_v4f o[NI];                                 // O rows 4 g4 + r, columns 64 q + 4 l16 + c of tile 4 q + c
 #pragma unroll
     for (int dt = 0; dt < NI; dt++) o[dt] = omh_v4f{0.f, 0.f, 0.f, 0.f};
 
     auto step = [&](int b) __attribute__((always_inline)) {
-        // scores of keys kb + 4 g4 + r for head l16 (two product chains)
+        // scores of keys kb + 4 g4 + r for column l16 (two product chains)
         omh_v4f sa = omh_v4f{0.f, 0.f, 0.f, 0.f}, sb = sa;
 #pragma unroll
         for (int i = 0; i < NI; i++) {
@@ -550,24 +580,25 @@ void attn_split_mfma_kernel(const AttnArgs a) {
         float sc[4], mx = -INFINITY;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            sc[r] = kb + 4 * g4 + r < k1 ? (sa[r] + sb[r]) * a.scale : -INFINITY;   // qwen.c:410-414
+            sc[r] = kb + 4 * g4 + r < kend ? (sa[r] + sb[r]) * a.scale : -INFINITY;   // qwen.c:410-414
             mx = fmaxf(mx, sc[r]);
         }
         mx = omh_swap32_max(omh_swap16_max(mx));
         // online softmax (qwen.c:413 softmax_ over all keys, merged per block);
-        // the block's first key is visible, so mn is finite
-        const float mn = fmaxf(m, mx);
-        const float corr = expf(m - mn);
+        // a decode step's blocks begin with a visible key, so mn is finite;
+        // with more tokens an early one may have seen none yet (weights 0)
+        const float mn = fmaxf(m, mx), ref = PREP || mn > -INFINITY ? mn : 0.f;
+        const float corr = expf(m - ref);
         float pr[4], ps = 0.f;
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-            pr[r] = kb + 4 * g4 + r < k1 ? expf(sc[r] - mn) : 0.f;
+            pr[r] = kb + 4 * g4 + r < kend ? expf(sc[r] - ref) : 0.f;
             ps += pr[r];
         }
         ps = omh_swap32_sum(omh_swap16_sum(ps));
         l = l * corr + ps;
         m = mn;
-        // the output rows are heads 4 g4 + r: their corrections from lanes 4 g4 + r
+        // the output rows are columns 4 g4 + r: their corrections from lanes 4 g4 + r
         float cr[4];
 #pragma unroll
         for (int r = 0; r < 4; r++) cr[r] = __shfl(corr, 4 * g4 + r, OMH_WAVE);
@@ -575,6 +606,54 @@ void attn_split_mfma_kernel(const AttnArgs a) {
         for (int dt = 0; dt < NI; dt++)
 #pragma unroll
             for (int r = 0; r < 4; r++) o[dt][r] *= cr[r];
+        // A block that some of the tile's tokens see only in part, and whose
+        // values are not all finite: a weight of zero would not hide those
+        // from the tokens before them, so this block's sums run key by key
+        // over the keys each column sees, O in the wave's LDS rows meanwhile.
+        if constexpr (!PREP) {
+            if (kb + 15 > a.pos) {
+                bool odd = false;
+#pragma unroll
+                for (int i = 0; i < NI; i++)
+#pragma unroll
+                    for (int c = 0; c < 4; c++) odd |= !(fabsf(kv[i][c]) < INFINITY);
+                if (__ballot(odd)) {
+                    float *ow = mo + wave * 16 * HD;
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++)
+                            *reinterpret_cast<omh_v4f *>(ow + (4 * g4 + r) * HD + 64 * q + 4 * l16) =
+                                omh_v4f{o[4 * q][r], o[4 * q + 1][r], o[4 * q + 2][r], o[4 * q + 3][r]};
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll 1
+                    for (int c = 0; c < ncol; c++) {
+                        const int ke = min(kb + 16, min(k1, a.pos + token_of(c0 + c) + 1)), d = 4 * lane % HD;
+                        omh_v4f acc = *reinterpret_cast<const omh_v4f *>(ow + c * HD + d);
+#pragma unroll 1
+                        for (int k = kb; k < ke; k++) {
+                            const int r = (k - kb) % 4;
+                            const float w = __shfl(r < 2 ? (r ? pr[1] : pr[0]) : (r > 2 ? pr[3] : pr[2]), (k - kb) / 4 * 16 + c, OMH_WAVE);
+                            acc += w * ld_buf_v4<false>(vrs, (k * HD + d) * 4);
+                        }
+                        __builtin_amdgcn_wave_barrier();     // (lanes past HD / 4 repeat the row)
+                        *reinterpret_cast<omh_v4f *>(ow + c * HD + d) = acc;
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
+                    __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                    for (int q = 0; q < NQ; q++)
+#pragma unroll
+                        for (int r = 0; r < 4; r++) {
+                            const omh_v4f x = *reinterpret_cast<const omh_v4f *>(ow + (4 * g4 + r) * HD + 64 * q + 4 * l16);
+#pragma unroll
+                            for (int c = 0; c < 4; c++) o[4 * q + c][r] = x[c];
+                        }
+                    return;
+                }
+            }
+        }
         // P.V (qwen.c:415-419)
 #pragma unroll
         for (int q = 0; q < NQ; q++)
@@ -590,7 +669,7 @@ void attn_split_mfma_kernel(const AttnArgs a) {
         step(b);
     }
 
-    // merge the waves: the workgroup's max per head, each wave's output scaled to it
+    // merge the waves: the workgroup's max per column, each wave's output scaled to it
     if (g4 == 0) {
         mm[wave * 16 + l16] = m;
         mm[NW * 16 + wave * 16 + l16] = l;
@@ -602,27 +681,29 @@ void attn_split_mfma_kernel(const AttnArgs a) {
         float M = -INFINITY;
 #pragma unroll
         for (int w = 0; w < NW; w++) M = fmaxf(M, mm[w * 16 + h]);
-        const float f = expf(mm[wave * 16 + h] - M);        // 0 for a wave without blocks (its m is -inf)
+        // 0 for a wave without blocks, or one whose column saw no key (its m is -inf)
+        const float f = PREP || M > -INFINITY ? expf(mm[wave * 16 + h] - M) : 0.f;
 #pragma unroll
         for (int q = 0; q < NQ; q++)
             *reinterpret_cast<omh_v4f *>(mo + (wave * 16 + h) * HD + 64 * q + 4 * l16) =
                 omh_v4f{o[4 * q][r] * f, o[4 * q + 1][r] * f, o[4 * q + 2][r] * f, o[4 * q + 3][r] * f};
     }
     __syncthreads();
-    for (int e = tid; e < grp * (HD / 4); e += NT) {
+    for (int e = tid; e < ncol * (HD / 4); e += NT) {
         const int i = e / (HD / 4), c = e % (HD / 4);
         omh_v4f acc = *reinterpret_cast<const omh_v4f *>(mo + i * HD + 4 * c);
 #pragma unroll
         for (int w = 1; w < NW; w++) acc += *reinterpret_cast<const omh_v4f *>(mo + (w * 16 + i) * HD + 4 * c);
-        *reinterpret_cast<omh_v4f *>(a.po + (pb + (size_t)i * ns) * HD + 4 * c) = acc;
+        *reinterpret_cast<omh_v4f *>(a.po + (row_of(i) * ns + s) * HD + 4 * c) = acc;
     }
-    if (tid < grp) {
+    if (tid < ncol) {
         float M = -INFINITY, L = 0.f;
 #pragma unroll
         for (int w = 0; w < NW; w++) M = fmaxf(M, mm[w * 16 + tid]);
+        if (PREP || M > -INFINITY)
 #pragma unroll
-        for (int w = 0; w < NW; w++) L += mm[NW * 16 + w * 16 + tid] * expf(mm[w * 16 + tid] - M);
-        const size_t pi = pb + (size_t)tid * ns;
+            for (int w = 0; w < NW; w++) L += mm[NW * 16 + w * 16 + tid] * expf(mm[w * 16 + tid] - M);
+        const size_t pi = row_of(tid) * ns + s;
         a.pml[2 * pi] = M;
         a.pml[2 * pi + 1] = L;
     }
@@ -1383,7 +1464,11 @@ hipError_t launch_attn_d(const AttnArgs &a, hipStream_t st) {
     // decode steps: the prep is done inside the split kernel (OMH_ATTN_FUSE=0: its own launch, for comparison)
     const bool flash = HD >= 128 && attn_uses_flash(a.T, HD);
     const bool fuse = a.T == 1 && !flash && fuse_prep();
-    if (!fuse) hipLaunchKernelGGL((attn_prep_kernel<HD>), dim3((unsigned)a.T), dim3(kPrepWaves * OMH_WAVE), 0, st, a);
+    // (few tokens: a token's rows over several workgroups, one row per wave)
+    if (!fuse) {
+        const int ny = a.T < 64 ? (a.H + 2 * a.KV + kPrepWaves - 1) / kPrepWaves : 1;
+        hipLaunchKernelGGL((attn_prep_kernel<HD>), dim3((unsigned)a.T, (unsigned)ny), dim3(kPrepWaves * OMH_WAVE), 0, st, a);
+    }
     if constexpr (HD >= 128) {
         if (attn_uses_flash(a.T, HD)) {
             if (flash_fp32()) {
@@ -1426,7 +1511,8 @@ hipError_t launch_attn_d(const AttnArgs &a, hipStream_t st) {
     if constexpr (HD >= 64) {
         // the K / V slices of a (sequence, kv head) are addressed by 32-bit byte offsets
         if ((size_t)a.max_t * HD * sizeof(float) > (size_t)INT32_MAX) return hipErrorInvalidValue;
-        const dim3 grid((unsigned)(a.ns * a.KV * a.T)), blk(MfmaSplitShape<HD>::NW * OMH_WAVE);
+        const int nct = (a.T * (a.H / a.KV) + 15) / 16;
+        const dim3 grid((unsigned)(a.ns * a.KV * nct)), blk(MfmaSplitShape<HD>::NW * OMH_WAVE);
         const size_t lds = MfmaSplitShape<HD>::LDS;
         if (fuse) hipLaunchKernelGGL((attn_split_mfma_kernel<HD, true>), grid, blk, lds, st, a);
         else hipLaunchKernelGGL((attn_split_mfma_kernel<HD, false>), grid, blk, lds, st, a);
@@ -1485,10 +1571,13 @@ bool attn_supported(int hd, int H, int KV, int rot) {
            H / KV <= kAttnMaxGroup && rot >= 0 && rot <= hd && rot % 2 == 0;
 }
 
-void attn_plan(int pos, int T, int KV, int &ns, int &kps) {
+void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
     const long nmax = (long)pos + T;                       // keys the last token sees
-    const long per = (long)KV * T;
-    const long want = per >= 256 ? 1 : (256 + per - 1) / per;   // splits for >= 256 workgroups (one per CU)
+    // workgroups per key split: a column tile of 16 (token, head) pairs each (width 32: a token each)
+    const long per = hd >= 64 ? (long)KV * (((long)T * (H / KV) + 15) / 16) : (long)KV * T;
+    // as many splits as leave every workgroup resident at once, one per CU
+    // (T = 5 at position 8001 with 260 workgroups, a token each: 47.7 us)
+    const long want = std::max(1L, 256 / per);
     long k = (nmax + want - 1) / want;
     k = (k + 63) / 64 * 64;
     kps = (int)k;

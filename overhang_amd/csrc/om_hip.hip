@@ -466,7 +466,7 @@ int attn_forward(int li, int seq, int pos, int T, const float *x, float *out, hi
     int ns = 0, kps = 0;
     const bool flash = attn_uses_flash(T, hd);
     if (flash) attn_flash_plan(pos, T, H, d.n_kv, hd, ns, kps);
-    else attn_plan(pos, T, d.n_kv, ns, kps);
+    else attn_plan(pos, T, H, d.n_kv, hd, ns, kps);
     const size_t nth = (size_t)T * H;
     if (int rc = ensure(g_arow, (size_t)T * A.rows * sizeof(float))) return rc;
     if (int rc = ensure(g_aqb, nth * hd * sizeof(float))) return rc;

@@ -357,3 +357,37 @@ def test_flash_key_splits(shape, pos, T, ramp):
         L.free()
     ref = q.gated_attention(x, _ref_w(w), [K.transpose(1, 0, 2)], [V.transpose(1, 0, 2)], pos, H, KV, hd, rot, 1e7, 1e-6)
     assert_close(got, ref, what=f"{shape} pos {pos} T {T} ramp {ramp}")
+
+
+@pytest.mark.parametrize("shape,pos,T", [(Q35B_ATTN, 0, 2), (Q35B_ATTN, 8001, 5), (Q35B_ATTN, 126, 17), (Q35B_ATTN, 1021, 63),
+                                         ((256, 8, 8, 32, 32), 100, 9), ((768, 6, 2, 64, 32), 333, 7),
+                                         ((512, 16, 1, 128, 128), 70, 3), ((1024, 4, 4, 256, 256), 511, 18)],
+                         ids=["pos0-T2", "pos8001-T5", "pos126-T17", "pos1021-T63", "hd32-T9", "hd64-grp3-T7", "hd128-grp16-T3",
+                              "hd256-grp1-T18"])
+@pytest.mark.parametrize("odd", [None, np.inf, np.nan], ids=["finite", "inf", "nan"])
+def test_few_token_steps(shape, pos, T, odd):
+    """Steps of 2 to 63 tokens share the key splits in column tiles of 16
+    (token, head) pairs: groups that fill a tile, that do not divide it, and
+    tiles whose last one is ragged, over splits whose keys only some of a
+    tile's tokens see.  A token whose input is not finite spoils itself and
+    the tokens after it, none before."""
+    D, H, KV, hd, rot = shape
+    rng = np.random.default_rng(43)
+    w = _weights(rng, D, H, KV, hd)
+    K = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32)
+    V = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32)
+    x = rng.normal(0, 1, (T, D)).astype(np.float32)
+    ref = q.gated_attention(x, _ref_w(w), [K.transpose(1, 0, 2)], [V.transpose(1, 0, 2)], pos, H, KV, hd, rot, 1e7, 1e-6)
+    first = T
+    if odd is not None:
+        first = T // 2
+        x[first, D // 3] = odd
+    L = gdn.AttnLayer(new_li(), D, H, KV, hd, rot, 1e7, 1e-6, pos + T, w)
+    try:
+        if pos:
+            L.cache_set(0, 0, pos, K, V)
+        got = L.forward(0, pos, x)
+    finally:
+        L.free()
+    assert_close(got[:first], ref[:first], what=f"{shape} pos {pos} T {T} {odd}")
+    assert not np.isfinite(got[first:]).any()
