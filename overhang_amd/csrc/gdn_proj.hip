@@ -1034,7 +1034,9 @@ void proj_q8_wave_kernel(const ProjArgs p, int nb, const F32Part f) {
 // are numbered token tile fastest and dealt out so that one XCD runs the
 // token tiles of a row group back to back: workgroups go to the XCDs in turn
 // (workgroup i to XCD i mod 8), so tile (i mod 8) * per + i / 8 keeps a row
-// group's weights in one L2.
+// group's weights in one L2.  Weights come from the tiled copy where there is
+// one, 1 KiB runs per load instead of 16 rows' 64-byte pieces: 150 tokens,
+// 9216 x 2048 27.5 -> 21.2 us, 2048 x 4096 22.1 -> 11.8 us.
 typedef int v4i __attribute__((ext_vector_type(4)));
 
 // x -> int8 planes with one scale per token (the power of two of the row's
@@ -1100,8 +1102,13 @@ void proj_split_i8_kernel(const float *__restrict__ x, int64_t ldx, int8_t *__re
 // row again, now from L2) into three 16-byte stores, so every store
 // instruction writes one contiguous 1 KiB run per plane.  (With 4 waves per
 // workgroup, one workgroup per CU, the loads' latency set the time: 29.7 us
-// for 4096 tokens of 2048.)
+// for 4096 tokens of 2048.)  Below kSplitTileMinT tokens there are too few
+// tiles for the CUs, and a workgroup per token is the faster: x of 2048 and
+// 4096 at 150 tokens 4.4 + 5.3 us against 8.1 + 14.7, at 700 6.2 + 9.2 against
+// 9.1 + 15.5; at 1500 10.3 + 18.4 against 11.2 + 17.4 and the GEMM after it 5 %
+// slower, at 4096 30.9 + 56.5 against 17.7 + 28.8.
 constexpr int kSplitTileWaves = 16;
+constexpr int kSplitTileMinT = 1024;
 __global__ __launch_bounds__(kSplitTileWaves * OMH_WAVE)
 void proj_split_i8_tile_kernel(const float *__restrict__ x, int64_t ldx, int8_t *__restrict__ xb, int T, int I) {
     __shared__ int s_e[16];
@@ -1197,7 +1204,10 @@ void proj_i8_kernel(const ProjArgs p, int nb, const F32Part f, int nrg, int ntt,
     const int8_t *xp[TT];
     const float *sp[TT];
 #pragma unroll
-    for (int rw = 0; rw < RW; rw++) wp[rw] = p.Q + (size_t)min(r0 + 16 * rw + l16, p.O - 1) * p.I + 16 * gq;
+    for (int rw = 0; rw < RW; rw++)
+        wp[rw] = p.Qt ? p.Qt + (size_t)min(r0 / 16 + rw, (p.O + 15) / 16 - 1) * (p.I / 64) * 1024 + 16 * lane
+                      : p.Q + (size_t)min(r0 + 16 * rw + l16, p.O - 1) * p.I + 16 * gq;
+    const int wh = p.Qt ? 1024 : 64;                              // bytes from a half block to the next
 #pragma unroll
     for (int tt = 0; tt < TT; tt++) {
         const int u = min(t0 / 16 + tt, i8_tiles(p.T) - 1);       // token tile
@@ -1214,7 +1224,7 @@ void proj_i8_kernel(const ProjArgs p, int nb, const F32Part f, int nrg, int ntt,
         for (int rw = 0; rw < RW; rw++)
 #pragma unroll
             for (int h = 0; h < 2; h++)
-                wq[sl][rw][h] = *reinterpret_cast<const v4i *>(wp[rw] + (size_t)kb * kI8Blk + 64 * h);
+                wq[sl][rw][h] = *reinterpret_cast<const v4i *>(wp[rw] + (2 * kb + h) * wh);
 #pragma unroll
         for (int tt = 0; tt < TT; tt++) {
 #pragma unroll
@@ -1390,7 +1400,9 @@ void proj_i8_kernel(const ProjArgs p, int nb, const F32Part f, int nrg, int ntt,
 // row scale combine once at the end, as in proj_i8_kernel's per-token form.
 // Tiles go to the XCDs by token tile (XCD x takes token tiles x, x + 8, ..),
 // each XCD walking patches of 4 row blocks x its token tiles, so the
-// workgroups one XCD runs together share their weights and x in its L2.
+// workgroups one XCD runs together share their weights and x in its L2; or,
+// where token tiles spread unevenly (gemm_per_xcd), as equal runs of the
+// patches of 4 row blocks x all token tiles.
 constexpr int kGmRows = 256, kGmTok = 64;
 constexpr int kGmWFrags = kGmRows / 16, kGmXFrags = kI8Planes * kGmTok / 16;   // fragments of one k step
 constexpr int kGmStage = (kGmWFrags + kGmXFrags) * 1024;                       // bytes of one LDS stage
@@ -1401,19 +1413,20 @@ constexpr int kGmWgs = 256;                                                    /
 // (block i: XCD i % 8, the XCD's i / 8-th tile, below), and its copy stream
 // runs on across tiles, so the next tile's first steps load while the
 // current one finishes and stores its outputs.
-__device__ __forceinline__ bool gemm_tile(int i, int nrb, int ntt, int &R0, int &t0) {
+__device__ __forceinline__ bool gemm_tile(int i, int nrb, int ntt, int even, int &R0, int &t0) {
     const int xcd = i % 8, j = i / 8;
-    const int nx = (ntt - xcd + 7) / 8;                      // token tiles of this XCD
-    if (j >= nx * nrb) return false;
-    const int grp = j / (4 * nx), rem = j % (4 * nx);
+    const int nx = even ? ntt : (ntt - xcd + 7) / 8;         // token tiles of a patch
+    const int q = even ? xcd * even + j : j;                 // place in the patches' order
+    if ((even && j >= even) || q >= nx * nrb) return false;
+    const int grp = q / (4 * nx), rem = q % (4 * nx);
     const int gr = min(4, nrb - 4 * grp);                    // row blocks in this patch
     R0 = (4 * grp + rem % gr) * kGmRows;
-    t0 = (xcd + 8 * (rem / gr)) * kGmTok;
+    t0 = (even ? rem / gr : xcd + 8 * (rem / gr)) * kGmTok;
     return true;
 }
 
 __global__ __launch_bounds__(8 * OMH_WAVE, 1)
-void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt) {
+void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt, int even) {
     // four stages, separate arrays, so each stage's copies and reads are
     // told apart by the compiler (its waits for this wave's copies into a
     // stage then cover only that stage)
@@ -1430,7 +1443,7 @@ void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt) {
     int NTL = 0;                                             // this workgroup's tiles
     {
         int r, t;
-        while (gemm_tile(b0 + G * NTL, nrb, ntt, r, t)) NTL++;
+        while (gemm_tile(b0 + G * NTL, nrb, ntt, even, r, t)) NTL++;
     }
     if (NTL == 0) return;
     const int NG = NTL * S;                                  // k steps over all of its tiles
@@ -1464,14 +1477,14 @@ void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt) {
     // the end: the last step again, unused); the stream runs in order, so the
     // tile's rows and tokens are worked out once per tile
     int ck = 0, cs = 0, cR0 = 0, ct0 = 0;
-    gemm_tile(b0, nrb, ntt, cR0, ct0);
+    gemm_tile(b0, nrb, ntt, even, cR0, ct0);
     auto copy = [&](auto st_c) __attribute__((always_inline)) {
         int8_t *dst = stage_of(st_c);
         const int R0 = cR0, t0 = ct0, s = cs;
         if (++cs == S) {
             if (ck + 1 < NTL) {
                 cs = 0;
-                gemm_tile(b0 + G * ++ck, nrb, ntt, cR0, ct0);
+                gemm_tile(b0 + G * ++ck, nrb, ntt, even, cR0, ct0);
             } else {
                 cs = S - 1;
             }
@@ -1522,7 +1535,7 @@ void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt) {
     // lane holds rows 4gq .. 4gq+3 of row fragment rw for token l16 of token tile tt
     auto store = [&](int k) __attribute__((always_inline)) {
         int R0, t0;
-        gemm_tile(b0 + G * k, nrb, ntt, R0, t0);
+        gemm_tile(b0 + G * k, nrb, ntt, even, R0, t0);
 #pragma unroll
         for (int tt = 0; tt < 2; tt++) {
             const int t = t0 + 32 * wt + 16 * tt + l16;
@@ -1603,31 +1616,56 @@ void proj_i8_gemm_kernel(const ProjArgs p, int nrb, int ntt) {
 }
 #undef OMH_LDS
 
+// Tiles of the XCD with the most, 8 XCDs of 32 CUs: by token tiles, or all
+// dealt out evenly (even > 0) where that takes fewer rounds of the CUs.  (By
+// token tiles 256 tokens sat on 4 XCDs: 9216 rows of 2048, 256 to 448 tokens
+// 47.3-48.0 us, evenly 26.0-29.2; 600 tokens 68.6 and 48.4.)
+int gemm_per_xcd(int nrb, int ntt, int &even) {
+    const int per = (ntt + 7) / 8 * nrb;
+    even = (ntt * nrb + 7) / 8;
+    if ((even + 31) / 32 < (per + 31) / 32) return even;
+    even = 0;
+    return per;
+}
+
 // The GEMM takes int8 rows with x split per token (not the decode core's
-// per-head planes) and the tiled copy of the weights, from kGmMinT tokens
+// per-head planes) and the tiled copy of the weights, above 64 tokens
 // (OMH_I8_GEMM=0 / 1 overrides, for tuning), with k a multiple of the loop
-// body's four 64-wide steps.
-constexpr int kGmMinT = 256;
-bool use_i8_gemm(const ProjArgs &p) {
+// body's four 64-wide steps, where it beats the kernel of 64-row tiles
+// (f32_rows: whose launch also takes a few fp32 rows, a launch of its own of
+// 10 us beside the GEMM).  The two estimates are fits in us to both kernels'
+// times: 9216 x 2048 at 150 / 256 / 448 tokens 21 / 34 / 53 against a GEMM
+// round of 26-29; 2048 x 4096 at 256 / 600 / 900 tokens 13 / 34 / 58 against
+// 40-44; 2560 x 1024 at 500 / 1000 tokens 17 / 26 against 16 / 18; 1024 x
+// 2048 at 1000 / 2000 tokens 13 / 26 against 16 / 17.
+bool use_i8_gemm(const ProjArgs &p, bool f32_rows) {
     if (p.x_split || !p.Qt || p.I % 256 != 0 || p.I > (1 << 25) / 127) return false;
     // (buffer offsets are 32-bit)
     if (tile_q8_bytes(p.O, p.I) >= (1u << 31) || kI8Planes * i8_plane_bytes(p.T, p.I) >= (1u << 31)) return false;
     if (const char *e = getenv("OMH_I8_GEMM")) return e[0] == '1';
-    return p.T >= kGmMinT;
+    if (p.T <= 64) return false;
+    if (p.I > 4096) return p.T >= 256;           // (the other kernel combines the planes block by block there)
+    const float K = p.I / 1024.f;
+    const float tiles = (float)((p.O + kI8Rows - 1) / kI8Rows) * ((p.T + 31) / 32);   // of 64 rows x 32 tokens
+    int even;
+    const int rounds = (gemm_per_xcd((p.O + kGmRows - 1) / kGmRows, (p.T + kGmTok - 1) / kGmTok, even) + 31) / 32;
+    return tiles / 256 * (2.4f * K + 3) > 8 * K * rounds + 6 + (f32_rows ? 10 : 0);
 }
 
 void launch_i8_gemm(const ProjArgs &p, hipStream_t st) {
     const int nrb = (p.O + kGmRows - 1) / kGmRows, ntt = (p.T + kGmTok - 1) / kGmTok;
-    const int per = (ntt + 7) / 8 * nrb;                     // tiles of the XCD with the most
+    int even;
+    const int per = gemm_per_xcd(nrb, ntt, even);
     // one resident workgroup per CU (LDS), each taking every 256th block
-    hipLaunchKernelGGL(proj_i8_gemm_kernel, dim3(std::min(8 * per, kGmWgs)), dim3(8 * OMH_WAVE), 0, st, p, nrb, ntt);
+    hipLaunchKernelGGL(proj_i8_gemm_kernel, dim3(std::min(8 * per, kGmWgs)), dim3(8 * OMH_WAVE), 0, st, p, nrb, ntt, even);
 }
 
 // Launch shape of the fp32-MFMA projection: one row tile per workgroup (k
 // split over its 4 waves) unless that leaves k-slices narrower than a
 // 64-wide block or far more workgroups than the device holds at once; a
 // few rows (e.g. the fp32 b / a rows beside int8 ones) take one token tile
-// per workgroup, so there are more of them.
+// per workgroup, so there are more of them (64 rows of 2048:
+// 2000 tokens 24.4 us in tiles of 64 and 22.1 in tiles of 16, 4096 24 and 37).
 struct F32Plan {
     int rt, tpw;
     dim3 grid;
@@ -2057,7 +2095,9 @@ void proj_i8_dq_kernel(const ProjArgs p, const F32Part f) {
 
 // Taken for 5..64 tokens of x split per token (not the decode core's
 // per-head planes) with the tiled weight copy, k a multiple of 128 kDqX and
-// the exact-int32 range (OMH_I8_DQ=0 turns it off, for comparison).
+// the exact-int32 range (OMH_I8_DQ=0 turns it off, for comparison).  Row tiles
+// per workgroup: 4 where that makes 128 workgroups, fewer below (2048 rows of
+// 4096, 40 tokens: 32 workgroups 13.8 us, 128 of one row tile 10.0).
 constexpr int kDqRT = 4;
 bool use_i8_dq(const ProjArgs &p) {
     if (p.T > 64 || p.T <= 4 || p.x_split || !p.Qt || p.I % (kI8Blk * kDqX) != 0 || p.I > (1 << 25) / 127) return false;
@@ -2066,10 +2106,14 @@ bool use_i8_dq(const ProjArgs &p) {
     return true;
 }
 void launch_i8_dq(const ProjArgs &p, const F32Part &f, hipStream_t st) {
-    const int nrg = (p.O + 16 * kDqRT - 1) / (16 * kDqRT);
-    const dim3 grid(f.nwg + nrg), blk(8 * OMH_WAVE);
-    if (p.I == 16 * kI8Blk) hipLaunchKernelGGL((proj_i8_dq_kernel<kDqRT, 16>), grid, blk, 0, st, p, f);
-    else hipLaunchKernelGGL((proj_i8_dq_kernel<kDqRT, 0>), grid, blk, 0, st, p, f);
+    const int tiles = (p.O + 15) / 16;
+    const int rt = tiles >= 128 * kDqRT ? kDqRT : tiles >= 256 ? 2 : 1;
+    const dim3 grid(f.nwg + (tiles + rt - 1) / rt), blk(8 * OMH_WAVE);
+#define OMH_DQ(RT)                                                                                          \
+    if (p.I == 16 * kI8Blk) hipLaunchKernelGGL((proj_i8_dq_kernel<RT, 16>), grid, blk, 0, st, p, f);         \
+    else hipLaunchKernelGGL((proj_i8_dq_kernel<RT, 0>), grid, blk, 0, st, p, f);
+    if (rt == kDqRT) { OMH_DQ(kDqRT) } else if (rt == 2) { OMH_DQ(2) } else { OMH_DQ(1) }
+#undef OMH_DQ
 }
 
 // Plan of the streaming kernel: T <= 64 tokens, RT row tiles per workgroup,
@@ -2560,7 +2604,7 @@ hipError_t launch_proj(const ProjArgs &p, hipStream_t st) {
         const int nclear = own ? 0 : lay.ncnt;
         const bool i8 = use_i8(p.T, p.I, p.n_q);
         // (planes written by the decode core: no split, unless counters need clearing)
-        if (i8 && !p.x_split && p.T > 64) {
+        if (i8 && !p.x_split && p.T >= kSplitTileMinT) {
             hipLaunchKernelGGL(proj_split_i8_tile_kernel, dim3((unsigned)i8_tiles(p.T)), dim3(kSplitTileWaves * OMH_WAVE), 0, st, p.x, p.ldx,
                                reinterpret_cast<int8_t *>(p.xb), p.T, p.I);
             if (nclear > 0)
@@ -2594,7 +2638,7 @@ hipError_t launch_proj(const ProjArgs &p, hipStream_t st) {
         } else if (sp.rt > 0) {
             launch_i8_stream(q, sp, fs, st);
             f32_done = nf32 > 0;
-        } else if (i8 && use_i8_gemm(q)) launch_i8_gemm(q, st);
+        } else if (i8 && use_i8_gemm(q, p.O > p.n_q)) launch_i8_gemm(q, st);
         else if (done && i8) launch_i8(q, lay.w, p.O > p.n_q ? &f : nullptr, &f32_done, st);
         else if (done) launch_q8_wave(q, lay.w, p.O > p.n_q ? &f : nullptr, &f32_done, st);
         if (!done) {

@@ -391,3 +391,13 @@ def test_few_token_steps(shape, pos, T, odd):
         L.free()
     assert_close(got[:first], ref[:first], what=f"{shape} pos {pos} T {T} {odd}")
     assert not np.isfinite(got[first:]).any()
+
+
+@pytest.mark.parametrize("shape", [Q35B_ATTN, (1024, 8, 2, 128, 64), (512, 4, 2, 64, 32)], ids=["35b", "k1024", "k512-k256"])
+@pytest.mark.parametrize("T", [17, 40, 64, 65, 160, 257, 449, 1023, 1025])
+def test_int8_projections_by_token_count(shape, T):
+    """The int8 projections around the lines of their dispatch: the queue
+    kernel's 1, 2 or 4 row tiles per workgroup (to 64 tokens), the 64-row
+    tiles from the tiled weights and the GEMM above, its tiles dealt out by
+    token tile or evenly, x split by token (below 1024) or by tile."""
+    _run(shape, [T], seed=13, int8=True)
