@@ -198,6 +198,12 @@ __device__ __forceinline__ void lower_tile(int it, int &i, int &j) {
     j = it - i * (i + 1) / 2;
 }
 
+// Value heads per WY item: two share the products of q and k, one where that
+// still leaves every item a CU of its own (32 value heads on 16 key heads, 150
+// tokens: 48 items of two 29.8 us, 96 of one 22.5; 512 tokens, 128 and 256:
+// 30.8 and 24.7).
+__host__ __device__ inline int wy_heads(int kh, int rep, int nc) { return rep % 2 == 0 && kh * rep * nc > 256 ? 2 : 1; }
+
 // Work item m -> (key head hk, first value head h0, chunk c) for items of
 // vpg value heads each (ngrp groups per key head), XCD-aware: with N items
 // and a grid that is a multiple of 8, the items a given XCD processes
@@ -384,7 +390,7 @@ void prefill_wy_kernel(const PrefillArgs a) {
     constexpr int NST = ScanShape<D>::NST;
 
     const int kh = a.kh, rep = a.vh / kh, nc = a.nc;
-    const int vpg = rep % 2 == 0 ? 2 : 1;                // value heads per item
+    const int vpg = wy_heads(kh, rep, nc);               // value heads per item
     const int nitems = kh * (rep / vpg) * nc;
     const int tid = threadIdx.x, lane = tid % OMH_WAVE;
     const int wave = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
@@ -1001,9 +1007,9 @@ void prefill_scan_kernel(const PrefillArgs a) {
 // Up to kFewTokens tokens (a speculative step's draft, a short turn): the
 // recurrence itself, one token after another, in one launch.  A 64-token
 // chunk costs its WY item, its scan step and two more launches however few of
-// its tokens are live (35B, any T <= 64: 28.9 + 7.4 + 4.1 us); one token of
-// the recurrence costs 0.5 us here, on top of 6 us for the launch, the state's
-// loads and the conv.  What bounds it is that chain: each SIMD runs two waves'
+// its tokens are live (35B core step, 33 to 64 tokens: 31.5-32.4 us); here 32
+// tokens take 30.7 us, 36 34.4 and 40 37.5, the launch, the state's loads and
+// the conv 6 us of it.  What bounds it is that chain: each SIMD runs two waves'
 // products of one token (128 a lane), then the lane sums.
 //
 // One workgroup per value head.  Wave w holds the state's columns 16 w .. +15
@@ -1017,7 +1023,7 @@ void prefill_scan_kernel(const PrefillArgs a) {
 // The conv history: a q / k channel's is read by all rep value heads of the
 // key head, so the last of them to have read it (an arrival counter that it
 // resets) commits the new inputs; v channels are the workgroup's own.
-constexpr int kFewTokens = 40;
+constexpr int kFewTokens = 32;
 template <int D>
 struct FewShape {
     static constexpr int NW = D / 16, NT = NW * OMH_WAVE;   // one wave per 16 columns
@@ -1204,7 +1210,7 @@ hipError_t launch_prefill_d(const PrefillArgs &a, hipStream_t st) {
     // persistent: one workgroup per CU (the LDS footprint allows one), a
     // multiple of 8 so the XCD-aware item order holds
     const int rep = a.vh / a.kh;
-    const int nitems = a.kh * (rep % 2 == 0 ? rep / 2 : rep) * a.nc;   // as in the kernel
+    const int nitems = a.kh * (rep / wy_heads(a.kh, rep, a.nc)) * a.nc;
     const int grid = nitems < wy_grid() ? nitems : wy_grid();
     // the WY kernel reads the ring for chunk 0 before the commit (in the
     // norm launch) rewrites it

@@ -300,9 +300,9 @@ def test_long_warm_append_35b_split_invariance(split):
 
 
 @pytest.mark.parametrize("kh,vh,D,K", [(2, 4, 16, 4), (1, 3, 32, 4), (2, 2, 64, 3), (2, 8, 128, 4), (1, 2, 128, 2)])
-@pytest.mark.parametrize("T", [2, 7, 8, 9, 17, 40, 41])
+@pytest.mark.parametrize("T", [2, 7, 8, 9, 17, 32, 33, 40])
 def test_few_token_prefill(kh, vh, D, K, T):
-    """Up to 40 tokens run the recurrence token by token in one launch, 41 and
+    """Up to 32 tokens run the recurrence token by token in one launch, 33 and
     more chunk-wise: two such steps in a row and a decode step, on the second
     of three sequences, so that the conv history each leaves (committed by the
     last value head of a key head to have read it) and its ring phase are
@@ -332,3 +332,24 @@ def test_few_token_prefill(kh, vh, D, K, T):
         r, _, _ = oracle.core_seq(d, w, *(one[k][s:s + 1] for k in ("qkv", "z", "a", "b")), c, S)
         assert_close(out[s:s + 1], r, what=what + f" decode of sequence {s}")
     L.free()
+
+
+@pytest.mark.parametrize("vh,T", [(8, 42), (8, 2048), (8, 2049), (6, 300)],
+                         ids=["1chunk", "256-chunk-heads", "264-chunk-heads", "3-heads-per-key-head"])
+def test_wy_items_of_one_or_two_value_heads(vh, T):
+    """A WY item is two value heads of a key head, or one while the (chunk,
+    value head) pairs are at most the CUs (256), as for an odd number of
+    heads per key head: both sides of that line."""
+    d = GdnDims(2, vh, 32, 32, 4, 0)
+    w = synth.layer_weights(d, 61, gnorm_std=0.1, projections=False)
+    conv0, S0 = synth.states(d, 61)
+    inp = synth.core_inputs(d, T, 61)
+    L = gdn.GdnLayer(new_li(), d, w)
+    L.set_state(0, conv0, S0)
+    got = L.prefill_core(0, *(inp[k] for k in ("qkv", "z", "a", "b")))
+    conv, S = L.get_state(0)
+    L.free()
+    ref, cref, Sref = oracle.core_seq(d, w, inp["qkv"], inp["z"], inp["a"], inp["b"], conv0, S0)
+    assert_close(got, ref, what=f"vh {vh} T {T} core")
+    assert_close(S, Sref, what=f"vh {vh} T {T} S")
+    assert np.array_equal(conv, cref)
