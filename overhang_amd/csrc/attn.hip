@@ -1571,13 +1571,13 @@ bool attn_supported(int hd, int H, int KV, int rot) {
            H / KV <= kAttnMaxGroup && rot >= 0 && rot <= hd && rot % 2 == 0;
 }
 
-void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
+void attn_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps) {
     const long nmax = (long)pos + T;                       // keys the last token sees
     // workgroups per key split: a column tile of 16 (token, head) pairs each (width 32: a token each)
     const long per = hd >= 64 ? (long)KV * (((long)T * (H / KV) + 15) / 16) : (long)KV * T;
     // as many splits as leave every workgroup resident at once, one per CU
     // (T = 5 at position 8001 with 260 workgroups, a token each: 47.7 us)
-    const long want = std::max(1L, 256 / per);
+    const long want = std::clamp(256 / per, 1L, most);
     long k = (nmax + want - 1) / want;
     k = (k + 63) / 64 * 64;
     kps = (int)k;
@@ -1589,7 +1589,7 @@ void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
 // sweep their tiles with kEnds tiles' worth of prologue and epilogue, one per
 // CU at a time (two at head width 128); their partials are written and read
 // once at about 4 TB/s.  One split where the unsplit workgroups fill the chip.
-void attn_flash_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
+void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps) {
     constexpr int KT = 32, NW = 4, kMaxSplits = 64;
     constexpr double kEnds = 3, kBytesPerTile = 6.4e6;
     const long nt = ((long)pos + T + KT - 1) / KT;
@@ -1600,7 +1600,7 @@ void attn_flash_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
     ns = 1;
     kps = (int)(nt * KT);
     if (flash_fp32()) return;
-    for (int s = 1; s <= kMaxSplits && s <= nt; s++) {
+    for (int s = 1; s <= kMaxSplits && s <= nt && s <= most; s++) {
         const long tps = (nt + s - 1) / s;
         if ((nt + tps - 1) / tps != s) continue;              // the same split as an earlier s
         const double per = s == 1 ? 1 : std::min((double)s, avg / tps + 0.5);   // live splits of a workgroup

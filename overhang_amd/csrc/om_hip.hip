@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -465,9 +466,19 @@ int attn_forward(int li, int seq, int pos, int T, const float *x, float *out, hi
     const int D = d.hidden, hd = d.head_dim, H = d.n_heads;
     int ns = 0, kps = 0;
     const bool flash = attn_uses_flash(T, hd);
-    if (flash) attn_flash_plan(pos, T, H, d.n_kv, hd, ns, kps);
-    else attn_plan(pos, T, H, d.n_kv, hd, ns, kps);
     const size_t nth = (size_t)T * H;
+    auto plan = [&](long most) {
+        if (flash) attn_flash_plan(pos, T, H, d.n_kv, hd, most, ns, kps);
+        else attn_plan(pos, T, H, d.n_kv, hd, most, ns, kps);
+    };
+    plan(LONG_MAX);
+    // scratch cannot grow in a stream capture: there a step takes the splits
+    // that its partials have room for (an unsplit flash step needs none)
+    const long room = (long)std::min(g_apo.n / (nth * hd * sizeof(float)), g_apml.n / (nth * 2 * sizeof(float)));
+    if (ns > room && (room > 0 || flash)) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) plan(std::max(1L, room));
+    }
     if (int rc = ensure(g_arow, (size_t)T * A.rows * sizeof(float))) return rc;
     if (int rc = ensure(g_aqb, nth * hd * sizeof(float))) return rc;
     if (int rc = ensure(g_actx, nth * hd * sizeof(float))) return rc;

@@ -229,10 +229,10 @@ bool attn_supported(int hd, int H, int KV, int rot);
 size_t attn_flash_image_bytes(int hd, int KV, int pos, int T, int *tiles);
 // whether a prompt step of T tokens runs on the flash kernel (no split partials)
 bool attn_uses_flash(int T, int hd);
-// splits for pos + T visible keys: workgroups for one round of the device's CUs where the keys allow
-void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps);
+// splits for pos + T visible keys, at most `most` >= 1: workgroups for one round of the device's CUs where the keys allow
+void attn_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps);
 // the same for a prompt step on the flash kernel (kps whole 32-key tiles; ns = 1: no partials)
-void attn_flash_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps);
+void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps);
 hipError_t launch_attn(const AttnArgs &a, int hd, hipStream_t st);
 
 // Returns hipSuccess, or hipErrorInvalidValue for an unsupported shape.

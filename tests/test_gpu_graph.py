@@ -13,6 +13,7 @@ import pytest
 
 from overhang_amd import gdn, hip, synth
 from overhang_amd.dims import CFG1, Q35B
+from tests.tol import assert_close
 
 pytestmark = pytest.mark.gpu
 
@@ -62,3 +63,40 @@ def test_graph_replays_equal_eager_decode(d, B, int8, nl):
         g.close()
         for L in A + E:
             L.free()
+
+
+@pytest.mark.parametrize("warm,pos,T", [(4096, 3072, 1024), (63, 3000, 40)], ids=["prompt", "few-tokens"])
+def test_captured_attention_step_takes_the_splits_its_scratch_has_room_for(warm, pos, T):
+    """Scratch cannot grow in a capture.  A first step from position 0 keeps
+    no partials, or those of one split; a captured step of fewer tokens behind
+    a long cache would split its keys further, and takes what fits instead.
+    Its replays match the eager step (which may grow the scratch) within the
+    contract: the same products summed in other splits."""
+    D, H, KV, hd, rot = 2048, 16, 2, 256, 64
+    rng = np.random.default_rng(47)
+    w = {"W_" + n: rng.normal(0, 0.02, s).astype(np.float32)
+         for n, s in {"q": (2 * H * hd, D), "k": (KV * hd, D), "v": (KV * hd, D), "o": (D, H * hd)}.items()}
+    w.update(q_norm=np.zeros(hd, np.float32), k_norm=np.zeros(hd, np.float32))
+    L = gdn.AttnLayer(3500, D, H, KV, hd, rot, 1e7, 1e-6, 4096, w, int8=True)
+    st = hip.Stream()
+    try:
+        L.cache_set(0, 0, pos, *(rng.normal(0, 1, (KV, pos, hd)).astype(np.float32) for _ in range(2)))
+        x = hip.Buffer.from_numpy(rng.normal(0, 1, (warm, D)).astype(np.float32))
+        out, eager = (hip.Buffer(warm * D * 4) for _ in range(2))
+        gdn.attn_forward_dev(L.li, 0, 0, warm, x, out, st)
+        st.synchronize()
+        g = hip.Graph(st, lambda: gdn.attn_forward_dev(L.li, 0, pos, T, x, out, st))
+        try:
+            got = []
+            for _ in range(3):
+                g.launch()
+                st.synchronize()
+                got.append(out.numpy((T, D)).copy())
+        finally:
+            g.close()
+        gdn.attn_forward_dev(L.li, 0, pos, T, x, eager, st)
+        st.synchronize()
+        for r, o in enumerate(got):
+            assert_close(o, eager.numpy((T, D)), what=f"replay {r}")
+    finally:
+        L.free()
