@@ -1357,8 +1357,7 @@ void attn_flash3_kernel(const AttnArgs a) {
         }
         return;
     }
-    // normalise and gate (qwen.c:420-421); the hardware sigmoid, because 128
-    // of the library's are 4000 instructions: 7 us at the end of a workgroup
+    // normalise and gate (qwen.c:420-421)
     const float il = 1.f / l;
     const float *gate = a.qkv + (size_t)tq * a.ld_qkv + (size_t)h * 2 * HD + HD + 4 * g2;
     float *dst = a.ctx + ((size_t)tq * H + h) * HD + 4 * g2;
@@ -1368,10 +1367,10 @@ void attn_flash3_kernel(const AttnArgs a) {
         for (int k = 0; k < 4; k++) {
             const float4 gv = *reinterpret_cast<const float4 *>(gate + 32 * d + 8 * k);
             float4 r;
-            r.x = o[d][4 * k] * il * omh_sigmoid_fast(gv.x);
-            r.y = o[d][4 * k + 1] * il * omh_sigmoid_fast(gv.y);
-            r.z = o[d][4 * k + 2] * il * omh_sigmoid_fast(gv.z);
-            r.w = o[d][4 * k + 3] * il * omh_sigmoid_fast(gv.w);
+            r.x = o[d][4 * k] * il * omh_sigmoid(gv.x);
+            r.y = o[d][4 * k + 1] * il * omh_sigmoid(gv.y);
+            r.z = o[d][4 * k + 2] * il * omh_sigmoid(gv.z);
+            r.w = o[d][4 * k + 3] * il * omh_sigmoid(gv.w);
             *reinterpret_cast<float4 *>(dst + 32 * d + 8 * k) = r;
         }
 }

@@ -11,10 +11,9 @@
 __device__ __forceinline__ float omh_sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
 __device__ __forceinline__ float omh_silu(float z) { return z * omh_sigmoid(z); }
 __device__ __forceinline__ float omh_softplus(float z) { return z > 20.f ? z : log1pf(expf(z)); }
-// Sigmoid and SiLU with the hardware exp2 and reciprocal (a few ulp; used
-// where they are evaluated for every channel of every token of a prompt).
-__device__ __forceinline__ float omh_sigmoid_fast(float z) { return __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
-__device__ __forceinline__ float omh_silu_fast(float z) { return z * omh_sigmoid_fast(z); }
+// SiLU with the hardware exp2 and reciprocal (a few ulp; used where it is
+// evaluated for every channel of every token of a prefill chunk).
+__device__ __forceinline__ float omh_silu_fast(float z) { return z * __builtin_amdgcn_rcpf(1.f + __expf(-z)); }
 
 // f(integral_constant<int, 0>) ... f(integral_constant<int, N-1>)
 template <int N, int I = 0, typename F>

@@ -401,3 +401,37 @@ def test_int8_projections_by_token_count(shape, T):
     tiles from the tiled weights and the GEMM above, its tiles dealt out by
     token tile or evenly, x split by token (below 1024) or by tile."""
     _run(shape, [T], seed=13, int8=True)
+
+
+@pytest.mark.parametrize("hd", [128, 256])
+@pytest.mark.parametrize("pos,T", [(0, 1), (100, 9), (0, 64), (2000, 64), (0, 300), (0, 1100)],
+                         ids=["decode", "few", "flash-T64", "flash-splits", "flash-images", "flash-T1100"])
+def test_output_gate_to_fp32_rounding(hd, pos, T):
+    """The output gate alone: keys of zero (every weight 1), values of one, so
+    the attention output is n / n = 1 for every token; gate logits that are
+    copies of x in [-30, 30] and an identity o_proj, whose other products are
+    exact zeros.  The result is sigmoid(x) within the roundings of fp32: 1 / n
+    and n (1 / n) (2 x 2^-24), expf (2^-23), 1 + e, the division and the
+    product with the output (3 x 2^-24): 3.5 x 2^-23 = 4.2e-7.  An exponent
+    rounded to fp32, |x| log2 e 2^-24, alone passes that below x = -10."""
+    H, KV = 2, 1
+    D = H * hd
+    rng = np.random.default_rng(53)
+    w = {"W_q": np.zeros((2 * D, D), np.float32), "W_k": np.zeros((KV * hd, D), np.float32),
+         "W_v": np.zeros((KV * hd, D), np.float32), "W_o": np.eye(D, dtype=np.float32),
+         "q_norm": np.zeros(hd, np.float32), "k_norm": np.zeros(hd, np.float32)}
+    src = 1 + np.arange(D) % (D - 1)                 # the input that is output i's gate logit
+    for h in range(H):
+        w["W_q"][2 * hd * h + hd + np.arange(hd), src[hd * h:hd * h + hd]] = 1.0
+    w["W_v"][:, 0] = 1.0
+    x = rng.uniform(-30, 30, (T, D)).astype(np.float32)
+    x[:, 0] = 1.0
+    L = gdn.AttnLayer(new_li(), D, H, KV, hd, 0, 1e7, 1e-6, pos + T, w)
+    try:
+        if pos:
+            L.cache_set(0, 0, pos, np.zeros((KV, pos, hd), np.float32), np.ones((KV, pos, hd), np.float32))
+        got = L.forward(0, pos, x)
+    finally:
+        L.free()
+    ref = 1.0 / (1.0 + np.exp(-x[:, src].astype(np.float64)))
+    assert_close(got, ref, atol=0.0, rtol=3.5 * 2.0**-23, what=f"hd {hd} pos {pos} T {T}")
