@@ -1574,13 +1574,13 @@ bool attn_supported(int hd, int H, int KV, int rot) {
            H / KV <= kAttnMaxGroup && rot >= 0 && rot <= hd && rot % 2 == 0;
 }
 
-void attn_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps) {
+void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
     const long nmax = (long)pos + T;                       // keys the last token sees
     // workgroups per key split: a column tile of 16 (token, head) pairs each (width 32: a token each)
     const long per = hd >= 64 ? (long)KV * (((long)T * (H / KV) + 15) / 16) : (long)KV * T;
     // as many splits as leave every workgroup resident at once, one per CU
     // (T = 5 at position 8001 with 260 workgroups, a token each: 47.7 us)
-    const long want = std::clamp(256 / per, 1L, most);
+    const long want = std::max(1L, 256 / per);
     long k = (nmax + want - 1) / want;
     k = (k + 63) / 64 * 64;
     kps = (int)k;
@@ -1599,6 +1599,7 @@ void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, 
     const long wpg = ((long)(T + 31) / 32 * (H / KV) + NW - 1) / NW;
     const double avg = 0.5 * ((double)nt + (double)(pos / KT + 1));   // tiles of a workgroup, unsplit
     const double slots = hd > 128 ? 256 : 512;
+    most = std::min(most, (long)(kFlashPartialBytes / ((size_t)T * H * hd * sizeof(float))));   // (0: unsplit)
     double best = 0;
     ns = 1;
     kps = (int)(nt * KT);

@@ -456,7 +456,7 @@ struct AttnLayer {
     float *Kc = nullptr, *Vc = nullptr;
 };
 AttnLayer g_A[kMaxLayers];
-Scratch g_arow, g_aqb, g_actx, g_apo, g_apml, g_aimg;
+Scratch g_arow, g_aqb, g_actx, g_apo, g_apml, g_fpart, g_aimg;
 
 void free_attn(AttnLayer &A) {
     void *ps[] = {A.Qin, A.Sin, A.Win, A.Qout, A.Sout, A.Wout, A.Qtin, A.Qtout, A.qn, A.kn, A.inv, A.Kc, A.Vc};
@@ -483,25 +483,32 @@ int attn_forward(int li, int seq, int pos, int T, const float *x, float *out, hi
     int ns = 0, kps = 0;
     const bool flash = attn_uses_flash(T, hd);
     const size_t nth = (size_t)T * H;
-    auto plan = [&](long most) {
-        if (flash) attn_flash_plan(pos, T, H, d.n_kv, hd, most, ns, kps);
-        else attn_plan(pos, T, H, d.n_kv, hd, most, ns, kps);
-    };
-    plan(LONG_MAX);
-    // scratch cannot grow in a stream capture: there a step takes the splits
-    // that its partials have room for (an unsplit flash step needs none)
-    const long room = (long)std::min(g_apo.n / (nth * hd * sizeof(float)), g_apml.n / (nth * 2 * sizeof(float)));
-    if (ns > room && (room > 0 || flash)) {
+    float *po = nullptr, *pml = nullptr;
+    if (flash) {
+        // the first flash step makes room for the partials of any split, so
+        // no later step moves them.  A step runs unsplit, without partials,
+        // where there is no memory for them or where it is captured (a
+        // capture cannot allocate) before any eager one has run.
+        long most = LONG_MAX;
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-        if (hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) plan(std::max(1L, room));
+        if (!g_fpart.p && hipStreamIsCapturing(st, &cap) == hipSuccess && cap == hipStreamCaptureStatusActive) most = 1;
+        if (most > 1 && ensure(g_fpart, kFlashPartialBytes + kFlashPartialBytes / 64) != OMH_OK) {
+            (void)hipGetLastError();
+            most = 1;
+        }
+        attn_flash_plan(pos, T, H, d.n_kv, hd, most, ns, kps);
+        po = static_cast<float *>(g_fpart.p);
+        if (po) pml = po + kFlashPartialBytes / sizeof(float);
+    } else {
+        attn_plan(pos, T, H, d.n_kv, hd, ns, kps);
+        if (int rc = ensure(g_apo, std::max(kSplitPartialBytes, nth * ns * hd * sizeof(float)))) return rc;
+        if (int rc = ensure(g_apml, std::max(kSplitPartialBytes / 16, nth * ns * 2 * sizeof(float)))) return rc;
+        po = static_cast<float *>(g_apo.p);
+        pml = static_cast<float *>(g_apml.p);
     }
     if (int rc = ensure(g_arow, (size_t)T * A.rows * sizeof(float))) return rc;
     if (int rc = ensure(g_aqb, nth * hd * sizeof(float))) return rc;
     if (int rc = ensure(g_actx, nth * hd * sizeof(float))) return rc;
-    if (!flash || ns > 1) {                           // (an unsplit flash step keeps no partials)
-        if (int rc = ensure(g_apo, nth * ns * hd * sizeof(float))) return rc;
-        if (int rc = ensure(g_apml, nth * ns * 2 * sizeof(float))) return rc;
-    }
     uint16_t *xb = nullptr;
     if (T > 4 && (A.nq > 0 || A.out_nq > 0)) {
         const size_t xbn = std::max(proj_xb_bytes(T, D, A.nq), proj_xb_bytes(T, A.qdim, A.out_nq));
@@ -522,8 +529,8 @@ int attn_forward(int li, int seq, int pos, int T, const float *x, float *out, hi
     a.qkv = rowb; a.ld_qkv = A.rows;
     a.qn = A.qn; a.kn = A.kn; a.inv = A.inv; a.Kc = A.Kc; a.Vc = A.Vc;
     a.qb = static_cast<float *>(g_aqb.p);
-    a.po = static_cast<float *>(g_apo.p);
-    a.pml = static_cast<float *>(g_apml.p);
+    a.po = po;
+    a.pml = pml;
     a.ctx = ctx;
     a.seq = seq; a.pos = pos; a.T = T; a.H = H; a.KV = d.n_kv; a.rot = d.rot_dim; a.max_t = d.max_t;
     a.ns = ns; a.kps = kps;

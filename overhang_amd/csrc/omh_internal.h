@@ -227,11 +227,23 @@ bool attn_supported(int hd, int H, int KV, int rot);
 // (keys 0 .. pos + T - 1 of each kv head; *tiles = tiles per kv head), or 0
 // (*tiles = 0) where its flash kernel stages tiles itself
 size_t attn_flash_image_bytes(int hd, int KV, int pos, int T, int *tiles);
-// whether a prompt step of T tokens runs on the flash kernel (no split partials)
+// whether a prompt step of T tokens runs on the flash kernel (partials only where attn_flash_plan gives ns > 1)
 bool attn_uses_flash(int T, int hd);
-// splits for pos + T visible keys, at most `most` >= 1: workgroups for one round of the device's CUs where the keys allow
-void attn_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps);
-// the same for a prompt step on the flash kernel (kps whole 32-key tiles; ns = 1: no partials)
+// Room for split partials, in bytes of partial outputs.  How many splits a
+// step takes neither rises nor falls with T or pos alone, so scratch that
+// grew with need could grow, and move, at any step, and a captured step would
+// then write into freed memory.  These bounds are reserved at once instead.
+// A flash step takes no more splits than fit (the largest that its estimate
+// asks for with 16 heads of 256: 94 MiB at up to 2048 tokens, 128 MiB for
+// 4096 tokens at position 16000); the other steps' splits make at most 256
+// workgroups of 16 rows, 4 MiB at width 256.  (Their bound is twice that:
+// what steps of the same sizes took with a workgroup per token.)  An unsplit
+// step of those needs T * H rows and grows with T, as the other scratch does.
+constexpr size_t kFlashPartialBytes = size_t(128) << 20;
+constexpr size_t kSplitPartialBytes = size_t(8) << 20;
+// splits for pos + T visible keys: workgroups for one round of the device's CUs where the keys allow
+void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps);
+// the same for a prompt step on the flash kernel, at most `most` (kps whole 32-key tiles; ns = 1: no partials)
 void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps);
 hipError_t launch_attn(const AttnArgs &a, int hd, hipStream_t st);
 
