@@ -417,6 +417,22 @@ struct MfmaSplitShape {
     static_assert(HD % 64 == 0, "64-column V groups");
 };
 
+// The token p / grp of (token, head) pair p without a division (five of them
+// before a step's first load cost 0.3 us): the high half of p times
+// r = ceil(2^32 / grp), exact while p (r grp - 2^32) < 2^32, so below 2^32 / 15
+// pairs; a cache of 2^31 bytes holds 2^23 tokens of width 64, 2^27 pairs.
+constexpr unsigned group_recip(int grp) { return grp > 1 ? 0xffffffffu / (unsigned)grp + 1 : 0; }
+__host__ __device__ constexpr int pair_token(int p, unsigned r) { return r ? (int)((uint64_t)(unsigned)p * r >> 32) : p; }
+constexpr bool pair_tokens_exact() {
+    for (int grp = 1; grp <= kAttnMaxGroup; grp++)
+        for (int t : {1, 2, 63, 155697, 339538, 1048576, (1 << 23) - 1}) {
+            const unsigned r = group_recip(grp);
+            if (pair_token(t * grp - 1, r) != t - 1 || pair_token(t * grp, r) != t || pair_token(t * grp + grp - 1, r) != t) return false;
+        }
+    return true;
+}
+static_assert(pair_tokens_exact(), "pair_token at the ends of a token's heads");
+
 // NT: streamed past the caches (one reader)
 template <bool NT>
 __device__ __forceinline__ omh_v4f ld_buf_v4(__amdgpu_buffer_rsrc_t r, int off) {
@@ -449,10 +465,9 @@ void attn_split_mfma_kernel(const AttnArgs a) {
     const int wave = __builtin_amdgcn_readfirstlane(tid / OMH_WAVE);
     const int l16 = lane % 16, g4 = lane / 16;
     // column c of the tile is (token, head) pair c0 + c of the group's
-    // T * grp, head fastest (the quotient by a reciprocal: fewer than 2^10
-    // pairs and 16 heads, so the half keeps every one clear of rounding)
-    const float rgrp = __builtin_amdgcn_rcpf((float)grp);
-    auto token_of = [&](int c) __attribute__((always_inline)) { return PREP ? 0 : (int)(((float)c + 0.5f) * rgrp); };
+    // T * grp, head fastest
+    const unsigned rgrp = PREP ? 0 : a.rgrp;
+    auto token_of = [&](int c) __attribute__((always_inline)) { return PREP ? 0 : pair_token(c, rgrp); };
     const int c0 = 16 * ct, ncol = PREP ? grp : min(16, a.T * grp - c0);
     const int tlast = token_of(c0 + ncol - 1);
     const int n = a.pos + tlast + 1;               // keys the tile's last token sees
@@ -1627,11 +1642,13 @@ hipError_t launch_attn(const AttnArgs &a, int hd, hipStream_t st) {
     if (!attn_supported(hd, a.H, a.KV, a.rot) || a.ns < 1 || a.kps < 1 || (long)a.ns * a.kps < (long)a.pos + a.T ||
         a.pos < 0 || (long)a.pos + a.T > a.max_t)
         return hipErrorInvalidValue;
+    AttnArgs b = a;
+    b.rgrp = group_recip(a.H / a.KV);
     switch (hd) {
-    case 32: return launch_attn_d<32>(a, st);
-    case 64: return launch_attn_d<64>(a, st);
-    case 128: return launch_attn_d<128>(a, st);
-    default: return launch_attn_d<256>(a, st);
+    case 32: return launch_attn_d<32>(b, st);
+    case 64: return launch_attn_d<64>(b, st);
+    case 128: return launch_attn_d<128>(b, st);
+    default: return launch_attn_d<256>(b, st);
     }
 }
 

@@ -221,6 +221,7 @@ struct AttnArgs {
     float eps, scale;                  // RMSNorm eps, hd^-1/2
     unsigned char *img;                // or null: the bf16 x 3 flash kernel's tile images [KV][img_tiles][tile]
     int img_tiles;                     //   (attn_flash_image_bytes), made in the same call from the cache
+    unsigned rgrp;                     // (set by launch_attn: ceil(2^32 / heads per kv head), 0 for one)
 };
 bool attn_supported(int hd, int H, int KV, int rot);
 // bytes of the tile images a prompt step of T tokens at position pos takes

@@ -393,6 +393,15 @@ def test_few_token_steps(shape, pos, T, odd):
     assert not np.isfinite(got[first:]).any()
 
 
+@pytest.mark.parametrize("H,KV,T", [(6, 2, 4097), (12, 1, 2500), (15, 1, 2999), (30, 2, 1025)],
+                         ids=["grp3", "grp12", "grp15", "grp15-kv2"])
+def test_long_steps_of_width_64(H, KV, T):
+    """Head width 64 has no flash kernel, so its steps of any length run as
+    column tiles: tens of thousands of (token, head) pairs in groups that do
+    not divide a tile."""
+    _run((256, H, KV, 64, 32), [7, T], seed=17)
+
+
 @pytest.mark.parametrize("shape", [Q35B_ATTN, (1024, 8, 2, 128, 64), (512, 4, 2, 64, 32)], ids=["35b", "k1024", "k512-k256"])
 @pytest.mark.parametrize("T", [17, 40, 64, 65, 160, 257, 449, 1023, 1025])
 def test_int8_projections_by_token_count(shape, T):
