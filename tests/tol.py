@@ -33,7 +33,7 @@ def assert_close(gpu, ref, atol=ATOL, rtol=RTOL, what=""):
     rel = float((err / np.maximum(np.abs(ref), 1e-30)).max()) if err.size else 0.0
     worst = float(ratio.max()) if err.size else 0.0
     MARGINS.append((_current_test(), what, mx, rel, worst))
-    bad = ratio > 1.0
+    bad = ~(ratio <= 1.0)                     # (a NaN on either side is no match)
     if bad.any():
         i = np.unravel_index(np.argmax(ratio), err.shape)
         raise AssertionError(f"{what}: {bad.sum()} of {bad.size} outside tolerance; worst at {i}: "
