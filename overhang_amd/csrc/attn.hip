@@ -124,6 +124,12 @@ __device__ __forceinline__ void prep_row(const AttnArgs &a, const float *src, co
     prep_row_regs<HD>(a, v, wv, w != nullptr, row, lane, cs_t, sn_t);
 }
 
+// Whether v is finite and rounds to a finite bf16; and where in a token's
+// projection row the prep leaves word of a v row (kv head g) that has a value
+// of which this is not so: at the row's own first element, copied by then.
+__device__ __forceinline__ bool bf16_finite(float v) { return fabsf(v) < 0x1.ffp127f; }
+__device__ __forceinline__ int odd_flag_at(int H, int KV, int g, int hd) { return (2 * H + KV + g) * hd; }
+
 // The prep: one workgroup of kPrepWaves waves per token (gridDim.y of them
 // where tokens are few, each with its share of the rows).  The token's RoPE
 // cos and sin (rot / 2 frequencies) go into LDS once, then wave w takes rows
@@ -180,6 +186,13 @@ __global__ __launch_bounds__(kPrepWaves * OMH_WAVE) void attn_prep_kernel(const 
         for (int i = 0; i < NE; i++) {
             const int j = lane + OMH_WAVE * i;
             if (j < HD) dst[j] = cv[i];
+        }
+        if (gridDim.y == 1 && r >= H + KV) {       // (flash steps among them)
+            bool odd = false;
+#pragma unroll
+            for (int i = 0; i < NE; i++) odd |= !bf16_finite(cv[i]);
+            const bool any = __builtin_amdgcn_ballot_w64(odd) != 0;
+            if (lane == 0) a.qkv[(size_t)t * a.ld_qkv + odd_flag_at(H, KV, r - H - KV, HD)] = any ? 1.f : 0.f;
         }
     }
 }
@@ -1106,6 +1119,19 @@ void attn_flash3_kernel(const AttnArgs a) {
     if (k0 >= k1) return;                          // (the merge reads no such split)
     const int kmax = a.pos + tq;                   // the last key this lane's token sees
 
+    // Values that are not finite must reach only the tokens that see them,
+    // and a weight of zero does not hide them from the others.  From key ka on
+    // the tiles hold keys that some of the workgroup's tokens do not see, rows
+    // of this step.  Where the prep left word that one of those is odd, the
+    // tiles from ka on are taken with such values as zeros, and at the end a
+    // token that sees one gets NaN in that dim.
+    const int ka = max(k0, (a.pos + 32 * (NW * wi / grp) + 1) / KT * KT);
+    const int kz = min(a.pos + a.T, (k1 + KT - 1) / KT * KT);
+    const float *Vk = a.Vc + (((size_t)a.seq * KV + g) * a.max_t + ka) * HD;
+    const int tf = max(ka - a.pos, 0) + lane;      // (requested ahead of q: their round trips overlap)
+    const float *flags = a.qkv + odd_flag_at(H, KV, g, HD);
+    float flag = flags[(size_t)min(tf, a.T - 1) * a.ld_qkv];
+
     // q as the B operand of S^T: dims 16 s + 8 g2 .. +7 of token tq, hi and lo
     omh_v8bf qh[NS], ql[NS];
     {
@@ -1118,6 +1144,9 @@ void attn_flash3_kernel(const AttnArgs a) {
             bf16_split8(v, qh[s], ql[s]);
         }
     }
+    flag = tf < kz - a.pos ? flag : 0.f;
+    for (int t = tf + OMH_WAVE; t < kz - a.pos; t += OMH_WAVE) flag += flags[(size_t)t * a.ld_qkv];   // (several token blocks)
+    const bool odd = __builtin_amdgcn_ballot_w64(flag != 0.f) != 0;   // (the same in every wave)
     const size_t cache0 = ((size_t)a.seq * KV + g) * a.max_t * HD;
     const float *Kg = a.Kc + cache0, *Vg = a.Vc + cache0;
     Flash3Frags<HD> fk, fv;
@@ -1152,6 +1181,24 @@ void attn_flash3_kernel(const AttnArgs a) {
     auto arrive = [&]() __attribute__((always_inline)) {
         if constexpr (IMG) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0): this wave's copies have landed
         __syncthreads();
+    };
+
+    // the V stage's values that are not finite as zeros: of the pieces that
+    // this wave has brought
+    auto scrub = [&](unsigned char *stage) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (int i = 0; i < F::VB / 1024 / NW; i++) {
+            const int c = IMG ? w + NW * i : 2 * (w + NW * (i / 2)) + i % 2;
+            uint32_t *p = reinterpret_cast<uint32_t *>(stage + c * 1024 + 16 * lane);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                uint32_t v = p[j];
+                if ((v & 0x7f80u) == 0x7f80u) v &= 0xffff0000u;
+                if ((v & 0x7f800000u) == 0x7f800000u) v &= 0xffffu;
+                p[j] = v;
+            }
+        }
+        __builtin_amdgcn_s_waitcnt(0xc07f);       // lgkmcnt(0): in place before the barrier that follows
     };
 
     omh_v16f o[ND];                                // O^T: o[d][i] = O[token tq][dim 32 d + 8 (i / 4) + 4 g2 + i % 4]
@@ -1308,6 +1355,10 @@ void attn_flash3_kernel(const AttnArgs a) {
     land_v(0);
     if (k0 + KT < k1) land_k(1);
     arrive();
+    if (odd && ka < k0 + KT) {
+        scrub(Vs);
+        __syncthreads();
+    }
     static_assert(NS % AHEAD == 0 && NS == 2 * ND && AHEAD % 2 == 0, "pairs in flight");
     constexpr int STEPS = NS / 2;
     omh_static_for<AHEAD>([&](auto i) { ask(Ks, i); });
@@ -1347,6 +1398,7 @@ void attn_flash3_kernel(const AttnArgs a) {
         // compiler leaves the wait for stores before a loop's back edge out
         // of the barrier at its head) have landed
         __builtin_amdgcn_s_waitcnt(IMG ? 0x0f70 : 0xc07f);
+        if (odd && ka < kt + 2 * KT) scrub(Vs + (st ^ 1) * F::VB);
     }
     if constexpr (F::EU == 1) acc_keep(o);
     __syncthreads();
@@ -1356,6 +1408,18 @@ void attn_flash3_kernel(const AttnArgs a) {
     if constexpr (F::EU == 1) acc_settle(o);
 
     if (!own || tq >= a.T) return;
+    // NaN over the dims of a written row in which its token sees a value that
+    // is not finite (after the row: o stays where the products left it)
+    auto mark = [&](float *row) __attribute__((always_inline)) {
+        if (!odd) return;
+#pragma unroll 1
+        for (int k = ka; k < min(kz, kmax + 1); k++)
+#pragma unroll 1
+            for (int d = 0; d < HD; d += 8)
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (!bf16_finite(Vk[(size_t)(k - ka) * HD + 4 * g2 + d + j])) row[d + j] = __builtin_nanf("");
+    };
     if (a.ns > 1) {
         // unnormalised partial of split sp (the reference in the scaled scores' units)
         const size_t pi = ((size_t)tq * H + h) * a.ns + sp;
@@ -1370,6 +1434,7 @@ void attn_flash3_kernel(const AttnArgs a) {
             a.pml[2 * pi] = m * a.scale;
             a.pml[2 * pi + 1] = l;
         }
+        mark(dst);
         return;
     }
     // normalise and gate (qwen.c:420-421)
@@ -1388,6 +1453,7 @@ void attn_flash3_kernel(const AttnArgs a) {
             r.w = o[d][4 * k + 3] * il * omh_sigmoid(gv.w);
             *reinterpret_cast<float4 *>(dst + 32 * d + 8 * k) = r;
         }
+    mark(dst);
 }
 
 // The flash kernel's splits merged, normalised and gated: a wave per (token,

@@ -209,7 +209,7 @@ hipError_t launch_state_copy(const StateCopyArgs &c, hipStream_t st);
 // seq at positions pos .. pos+T-1, after the qkv projection.
 constexpr int kAttnMaxGroup = 16;     // query heads per kv head
 struct AttnArgs {
-    const float *qkv; int64_t ld_qkv;  // [T] rows: H x (hd q, hd gate), KV x hd k, KV x hd v
+    float *qkv; int64_t ld_qkv;        // [T] rows: H x (hd q, hd gate), KV x hd k, KV x hd v (the prep reuses the v part)
     const float *qn, *kn;              // [hd] RMSNorm weights of q and k (applied as 1 + w)
     const float *inv;                  // [rot / 2] RoPE inverse frequencies
     float *Kc, *Vc;                    // [max_seqs][KV][max_t][hd] caches

@@ -393,6 +393,44 @@ def test_few_token_steps(shape, pos, T, odd):
     assert not np.isfinite(got[first:]).any()
 
 
+@pytest.mark.parametrize("shape,pos,T,first", [(Q35B_ATTN, 0, 64, 33), (Q35B_ATTN, 45, 100, 70), (Q35B_ATTN, 3000, 65, 1),
+                                               (Q35B_ATTN, 0, 300, 299), (Q35B_ATTN, 77, 515, 200), (Q35B_ATTN, 1500, 256, 31),
+                                               ((512, 16, 1, 128, 128), 9, 130, 111), ((512, 16, 1, 128, 128), 600, 300, 150),
+                                               ((1024, 4, 4, 256, 256), 5, 200, 100), ((1024, 4, 4, 256, 256), 640, 300, 64)],
+                         ids=["T64", "pos45-T100", "pos3000-T65", "T300", "pos77-T515", "pos1500-T256", "hd128-T130",
+                              "hd128-T300", "grp1-T200", "grp1-T300"])
+@pytest.mark.parametrize("odd", [np.inf, np.nan], ids=["inf", "nan"])
+def test_flash_steps_keep_odd_values_to_their_tokens(shape, pos, T, first, odd):
+    """A token of a flash step whose input is not finite spoils itself and the
+    tokens after it and none before, although those share its key tile (a
+    weight of zero times infinity is not zero): tiles staged by the kernel and
+    from images, with key splits and without, one and several tokens' blocks a
+    workgroup.  In a second step one value of the cache row before the step's,
+    in the tile of its first keys, is not finite: every token sees it."""
+    D, H, KV, hd, rot = shape
+    rng = np.random.default_rng(59)
+    w = _weights(rng, D, H, KV, hd)
+    K = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32)
+    V = rng.normal(0, 1, (KV, pos, hd)).astype(np.float32)
+    x = rng.normal(0, 1, (T, D)).astype(np.float32)
+    ref = q.gated_attention(x, _ref_w(w), [K.transpose(1, 0, 2)], [V.transpose(1, 0, 2)], pos, H, KV, hd, rot, 1e7, 1e-6)
+    bad = x.copy()
+    bad[first, D // 3] = odd
+    L = gdn.AttnLayer(new_li(), D, H, KV, hd, rot, 1e7, 1e-6, pos + T, w)
+    try:
+        if pos:
+            L.cache_set(0, 0, pos, K, V)
+        got = L.forward(0, pos, bad)
+        assert_close(got[:first], ref[:first], atol=2e-5, rtol=2e-4, what=f"{shape} pos {pos} T {T} before token {first}")
+        assert not np.isfinite(got[first:]).any()
+        if pos:
+            V[:, pos - 1, 7] = odd
+            L.cache_set(0, 0, pos, K, V)
+            assert not np.isfinite(L.forward(0, pos, x)).any()
+    finally:
+        L.free()
+
+
 @pytest.mark.parametrize("H,KV,T", [(6, 2, 4097), (12, 1, 2500), (15, 1, 2999), (30, 2, 1025)],
                          ids=["grp3", "grp12", "grp15", "grp15-kv2"])
 def test_long_steps_of_width_64(H, KV, T):
