@@ -1049,10 +1049,13 @@ __global__ __launch_bounds__(Flash3Shape<HD>::NW * OMH_WAVE) void attn_tile_imag
 }
 
 // The products of the one-wave-per-SIMD form, with its output in accumulation
-// registers and everything else in vector registers for the whole sweep:
-// through the builtin the compiler puts all results in accumulation registers
-// and moves 128 of them to vector registers and back on every tile.  It does
-// not see what these instructions are, so their waits are here: two states
+// registers for the whole sweep and everything else in vector registers (the
+// form that stages its tiles itself has about 50 values too many for those and
+// keeps them in accumulation registers between uses): through the builtin the
+// compiler puts all results in accumulation registers and moves 128 of them to
+// vector registers and back on every tile.  It does not see what these
+// instructions are, so their waits are here (test_flash_waits.py follows them
+// through the compiled code): two states
 // before each (an operand may just have been written by a VALU instruction,
 // a move between the register files among them; they pass while the product
 // before still runs), and acc_settle and vec_settle (a product's write lands
@@ -1669,10 +1672,13 @@ void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
 }
 
 // Key splits of a prompt step on the flash kernel, by an estimate of its time
-// in 32-key tiles of one workgroup (about 1.6 us): the workgroups of a split
-// sweep their tiles with kEnds tiles' worth of prologue and epilogue, one per
-// CU at a time (two at head width 128); their partials are written and read
-// once at about 4 TB/s.  One split where the unsplit workgroups fill the chip.
+// in 32-key tiles of one workgroup: the workgroups of a split sweep their
+// tiles with kEnds tiles' worth of prologue and epilogue, one per CU at a time
+// (two at head width 128); partials cost a tile per kBytesPerTile written and
+// read, and the merge two.  One split where the unsplit workgroups fill the
+// chip.  A tile is 2.8 us in a step of 333 tokens at position 6000 (5 splits of
+// 40 tiles, 119 us) and 3.6 us at 4096 tokens, where 6.4 MB a tile are 2.3 and
+// 1.8 TB/s: a price above what partials cost, on the side of fewer splits.
 void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps) {
     constexpr int KT = 32, NW = 4, kMaxSplits = 64;
     constexpr double kEnds = 3, kBytesPerTile = 6.4e6;
