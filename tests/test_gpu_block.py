@@ -13,7 +13,7 @@ import pytest
 import oracle
 from overhang_amd import gdn, synth
 from overhang_amd.dims import CFG1, TINY, Q35B, GdnDims
-from tests.tol import assert_close
+from tests.tol import assert_close, assert_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -248,7 +248,7 @@ def test_35b_int8_prefill_block_matches_oracle(T):
                          ids=["35b-T300", "kh3-T270"])
 def test_int8_gemm_matches_wave_kernel(shape, T, monkeypatch):
     """The prefill-sized int8 GEMM against the int8 wave-tile kernel it
-    replaces from 256 tokens (OMH_I8_GEMM forces either): both sum every
+    replaces where an estimate of both has it faster (OMH_I8_GEMM forces either): both sum every
     plane product exactly in int32, so the two layers agree to fp32
     rounding of the plane combine (kh3: 1152 in_proj int8 rows, not a
     multiple of the GEMM's 256-row tile; both: partial token tiles)."""
@@ -312,7 +312,9 @@ def test_few_token_projections(shape, int8, B):
     end inside a tile; tokens from 1e-3 to 10 in size, since each is scaled
     by its own largest value.  (The output grows with the gate silu(z), so with
     x: at 1e3 its rms is about 600 and fp32 sums in another order, 1e-5 of
-    that, pass the absolute 2e-3; at 10 they stay below 1e-4.)"""
+    that, pass the absolute 2e-3; at 10 they stay below 1e-4.)  Relative bound
+    per token: fp32 sums of up to 4096 products in another order, sqrt(4096)
+    2^-24 = 4e-6 in each of the two projections, above the 2^-22 of the split."""
     kh, vh, kd, vd, hidden = shape
     d = GdnDims(kh=kh, vh=vh, kd=kd, vd=vd, K=4, hidden=hidden)
     w = synth.layer_weights(d, 3)
@@ -331,3 +333,4 @@ def test_few_token_projections(shape, int8, B):
     for b in range(B) if kh < 16 else (0, 1, B - 1):
         ref, _, _ = oracle.layer_seq(d, w, x[b:b + 1], conv0[b], S0[b], int8=int8)
         assert_close(out[b:b + 1], ref, what=f"{shape} int8={int8} token {b} of {B}")
+        assert_rel(out[b:b + 1], ref, 1e-5, what=f"rel token {b}")

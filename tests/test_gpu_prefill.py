@@ -13,7 +13,7 @@ import oracle
 from overhang_amd import gdn, synth
 from overhang_amd.dims import GdnDims, Q35B, CFG1, TINY
 from tests import fixtures
-from tests.tol import assert_close
+from tests.tol import assert_close, assert_rel
 
 pytestmark = pytest.mark.gpu
 
@@ -306,8 +306,13 @@ def test_few_token_prefill(kh, vh, D, K, T):
     more chunk-wise: two such steps in a row and a decode step, on the second
     of three sequences, so that the conv history each leaves (committed by the
     last value head of a key head to have read it) and its ring phase are
-    taken up by the next and the other sequences are left as they were."""
+    taken up by the next and the other sequences are left as they were.
+    Relative bounds: token by token, fp32 sums over D values and up to 64
+    steps in another order than the oracle's, sqrt(64 D) 2^-24 = 5e-6 at 128;
+    chunk-wise those sums go through the inverse of a unit triangle of up to
+    64 rows, whose norm, up to 10 for these inputs, multiplies them."""
     d = GdnDims(kh, vh, D, D, K, 0)
+    rel = 1e-5 if T <= 32 else 5e-5
     seed = 5000 + 7 * kh + vh + D + K + T
     w = synth.layer_weights(d, seed, gnorm_std=0.1, projections=False)
     conv0, S0 = synth.states(d, seed)
@@ -319,10 +324,12 @@ def test_few_token_prefill(kh, vh, D, K, T):
     ref, cref, Sref = oracle.core_seq(d, w, inp["qkv"], inp["z"], inp["a"], inp["b"], conv0, S0)
     what = f"kh={kh} vh={vh} D={D} K={K} T={T}"
     assert_close(np.concatenate(got), ref, what=what + " core")
+    assert_rel(np.concatenate(got), ref, rel, what=what + " rel")
     for s in range(3):
         conv, S = L.get_state(s)
         if s == 1:
             assert_close(S, Sref, what=what + " S")
+            assert_rel(S, Sref, rel, what=what + " rel S")
             assert np.array_equal(conv, cref), "conv history is a copy of the inputs"
         else:
             assert np.array_equal(conv, conv0) and np.array_equal(S, S0), f"sequence {s} changed"

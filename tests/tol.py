@@ -39,3 +39,15 @@ def assert_close(gpu, ref, atol=ATOL, rtol=RTOL, what=""):
         raise AssertionError(f"{what}: {bad.sum()} of {bad.size} outside tolerance; worst at {i}: "
                              f"gpu={gpu[i]:.6g} ref={ref[i]:.6g} (max abs err {mx:.3g})")
     return mx
+
+
+def assert_rel(gpu, ref, rel, what=""):
+    """The 2-norm of the difference within `rel` of the reference's: the
+    rounding of a path's number formats, where the elementwise contract would
+    also pass a lost low-order term."""
+    gpu, ref = np.asarray(gpu, np.float64), np.asarray(ref, np.float64)
+    assert gpu.shape == ref.shape, (what, gpu.shape, ref.shape)
+    off, norm = float(np.linalg.norm(gpu - ref)), float(np.linalg.norm(ref))
+    got = off / norm if norm else (0.0 if off == 0 else np.inf)     # (a result of zeros has no error)
+    MARGINS.append((_current_test(), what, float(np.abs(gpu - ref).max()), got, got / rel))
+    assert got <= rel, f"{what}: relative error {got:.3g}, bound {rel:.3g}"
