@@ -1676,8 +1676,8 @@ void attn_plan(int pos, int T, int H, int KV, int hd, int &ns, int &kps) {
 // tiles with kEnds tiles' worth of prologue and epilogue, one per CU at a time
 // (two at head width 128); partials cost a tile per kBytesPerTile written and
 // read, and the merge two.  One split where the unsplit workgroups fill the
-// chip.  A tile is 2.8 us in a step of 333 tokens at position 6000 (5 splits of
-// 40 tiles, 119 us) and 3.6 us at 4096 tokens, where 6.4 MB a tile are 2.3 and
+// chip.  A tile is 2.5 us in a step of 333 tokens at position 6000 (5 splits of
+// 40 tiles, 107 us) and 3.6 us at 4096 tokens, where 6.4 MB a tile are 2.6 and
 // 1.8 TB/s: a price above what partials cost, on the side of fewer splits.
 void attn_flash_plan(int pos, int T, int H, int KV, int hd, long most, int &ns, int &kps) {
     constexpr int KT = 32, NW = 4, kMaxSplits = 64;
