@@ -145,22 +145,6 @@ int upload(T **dst, size_t count, const T *src) {
     return OMH_OK;
 }
 
-// A layer's state (the recurrent blocks, the conv ring): kernels touch
-// exactly these bytes, so a buffer of 1 MiB and more is whole 2 MiB pages
-// without the slack that upload() adds.  With those 16 bytes past its last
-// page a buffer of 17 slots (34 MiB) took 18 pages of address space, and the
-// time of a launch over 30 layers then hung on what else the process had
-// allocated before them: 23.7 to 24.3 us over a few placements, against
-// 23.4 to 23.8 in whole pages (16 slots: 23.4-23.6 and 23.35-23.45; 8 alike).
-int alloc_state(float **dst, size_t count) {
-    constexpr size_t kPage = size_t(2) << 20;
-    const size_t bytes = count * sizeof(float);
-    if (bytes < kPage / 2) return upload(dst, count, (const float *)nullptr);
-    if (hipMalloc(reinterpret_cast<void **>(dst), (bytes + kPage - 1) / kPage * kPage) != hipSuccess)
-        return fail(OMH_ERR_ALLOC, "alloc of %zu bytes of state failed", bytes);
-    return OMH_OK;
-}
-
 // The tiled copy of O x I int8 weights the prefill-sized GEMM reads
 // (tile_q8), where the shape takes one; *Qt stays null otherwise.
 int upload_tiled(int8_t **Qt, const int8_t *Q, int O, int I) {
@@ -614,10 +598,8 @@ int omh_gdn_layer_init(int li, const omh_gdn_dims *d, const omh_gdn_weights *w, 
     UP(L.gnorm, d->vd, w->gnorm);
     const size_t nring = (size_t)max_seqs * L.conv_dim * kConvRing;
     const size_t nS = (size_t)max_seqs * vh * d->kd * d->vd;
-    if ((rc = alloc_state(&L.conv_st, nring)) != OMH_OK || (rc = alloc_state(&L.S, nS)) != OMH_OK) {
-        free_layer(L);
-        return rc;
-    }
+    UP(L.conv_st, nring, (const float *)nullptr);
+    UP(L.S, nS, (const float *)nullptr);
     UP(L.phase, (size_t)2 * max_seqs, (const int *)nullptr);
     UP(L.o_raw, (size_t)max_seqs * L.vdim, (const float *)nullptr);
     UP(L.ssq, (size_t)max_seqs * vh * kMaxSlices, (const float *)nullptr);
