@@ -145,6 +145,24 @@ int upload(T **dst, size_t count, const T *src) {
     return OMH_OK;
 }
 
+// A layer's state (the recurrent blocks, the conv ring): kernels touch
+// exactly these bytes, so a buffer of 1 MiB and more is whole 2 MiB pages
+// without the slack that upload() adds (with those 16 bytes past its last
+// page, 17 slots, 34 MiB, take 18 pages).  How the layers' states lie to each
+// other sets a large launch's time, and what else the process has allocated
+// moves them.  17 slots a layer, one token, twelve heaps each, with the slack
+// and without, us: 30 layers 23.75-24.32 and 23.45-23.87, 22 layers 20.55-20.87
+// and 20.59-20.71, 15 layers 14.15-14.34 and 14.21-14.48, 11 layers 12.48-12.58
+// and 12.51-12.61, 8 layers 8.25-8.52 and 8.21-8.41.
+int alloc_state(float **dst, size_t count) {
+    constexpr size_t kPage = size_t(2) << 20;
+    const size_t bytes = count * sizeof(float);
+    if (bytes < kPage / 2) return upload(dst, count, (const float *)nullptr);
+    if (hipMalloc(reinterpret_cast<void **>(dst), (bytes + kPage - 1) / kPage * kPage) != hipSuccess)
+        return fail(OMH_ERR_ALLOC, "alloc of %zu bytes of state failed", bytes);
+    return OMH_OK;
+}
+
 // The tiled copy of O x I int8 weights the prefill-sized GEMM reads
 // (tile_q8), where the shape takes one; *Qt stays null otherwise.
 int upload_tiled(int8_t **Qt, const int8_t *Q, int O, int I) {
@@ -598,8 +616,10 @@ int omh_gdn_layer_init(int li, const omh_gdn_dims *d, const omh_gdn_weights *w, 
     UP(L.gnorm, d->vd, w->gnorm);
     const size_t nring = (size_t)max_seqs * L.conv_dim * kConvRing;
     const size_t nS = (size_t)max_seqs * vh * d->kd * d->vd;
-    UP(L.conv_st, nring, (const float *)nullptr);
-    UP(L.S, nS, (const float *)nullptr);
+    if ((rc = alloc_state(&L.conv_st, nring)) != OMH_OK || (rc = alloc_state(&L.S, nS)) != OMH_OK) {
+        free_layer(L);
+        return rc;
+    }
     UP(L.phase, (size_t)2 * max_seqs, (const int *)nullptr);
     UP(L.o_raw, (size_t)max_seqs * L.vdim, (const float *)nullptr);
     UP(L.ssq, (size_t)max_seqs * vh * kMaxSlices, (const float *)nullptr);
